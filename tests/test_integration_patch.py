@@ -24,7 +24,7 @@ def patched_files():
     return old, new
 
 
-@pytest.mark.skipif(not os.path.isdir(REF), reason="the reference tree is not present here")
+@pytest.mark.skipif(not os.path.isdir(os.path.join(REF, "src")), reason="the reference tree is not present here")
 def test_patch_applies_to_the_reference_files(tmp_path):
     old, new = patched_files()
     assert old, "the patch changes no existing file"
