@@ -46,6 +46,10 @@ SOURCES = {
     "qmv_mr.hip": [],
     "qmm_group.hip": [],
     "qmm.hip": [],
+    "qmm_strip.hip": [],
+    "qmm_strip_odd.hip": [],
+    "qmm_strip_f16.hip": [],
+    "qmm_strip_f16_odd.hip": [],
     "qmm_gen.hip": [],
     "moe.hip": [],
     "bias.hip": [],

@@ -575,6 +575,8 @@ struct Knobs {
   int kq_t = 0;    // its 16-row tiles per workgroup (1-4; 0: planner)
   int qmm_streamk = 1;  // prefill: stream-K plan for a part-full last round of 256 x 256 tiles (0: off)
   int sk_fallback = 0;  // stream-K: every cut tile's head computes its tail itself (tests)
+  int strip = 1;      // strip kernel: 0 off, 2 forced for every dense call it covers
+  int strip_nwn = 0, strip_mt = 0, strip_ks = 0;  // its waves along N, activation tiles, K ranges (0: planner)
   std::string qmv_kernel;  // "", "rs", "b4", "mid", "mr", "kq", "fr", "mfma"
 };
 
@@ -613,6 +615,10 @@ const Knobs* read_knobs() {
   k->kq_t = env_int("MLXQ_QMV_KQ_T", 0);
   k->qmm_streamk = env_int("MLXQ_QMM_STREAMK", 1);
   k->sk_fallback = env_int("MLXQ_QMM_SK_FALLBACK", 0);
+  k->strip = env_int("MLXQ_STRIP", 1);
+  k->strip_nwn = env_int("MLXQ_STRIP_NWN", 0);
+  k->strip_mt = env_int("MLXQ_STRIP_MT", 0);
+  k->strip_ks = env_int("MLXQ_STRIP_KS", 0);
   const char* v = std::getenv("MLXQ_QMV_KERNEL");
   k->qmv_kernel = v ? v : "";
   return k;
@@ -705,6 +711,12 @@ DirectIdx direct_index(const mlxq_array* idx, const Shape& dflt, const Shape& b)
   d.ok = true;
   d.div = (int)div;
   return d;
+}
+
+int gs_shift_of(int gs) {
+  int shift = 0;
+  while ((1 << shift) < gs) shift++;
+  return shift;
 }
 
 int fmt_of(Mode m, int bits) {
@@ -1295,6 +1307,89 @@ bool try_qmm_f16(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, co
   return true;
 }
 
+// Whether a call may take `bytes` of scratch without allocating under a
+// capture (or past the fixed scratch).
+bool scratch_fits(int dev, hipStream_t stream, size_t bytes, const ScratchSrc& ss) {
+  if (ss.fixed) return bytes <= ss.max;
+  {
+    std::lock_guard<std::mutex> lk(g_mu);
+    const auto it = g_ws.find({dev, stream, 0});
+    if (it != g_ws.end() && it->second.bytes >= bytes) return true;
+  }
+  return !stream_capturing(stream);
+}
+
+// Operands of the strip kernel: transpose=true; x, scales and biases all
+// bfloat16 or all float16 with affine codes of 2-6 or 8 bits, or bfloat16 x
+// with mxfp4.
+bool strip_types(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* scales, const mlxq_array* biases) {
+  if (!sp.transpose || !sp.small_w) return false;
+  const int dt = sp.out_dtype;
+  if ((dt != MLXQ_BFLOAT16 && dt != MLXQ_FLOAT16) || x->dtype != dt) return false;
+  if (sp.mode == AFFINE)
+    return biases && scales->dtype == dt && biases->dtype == dt && sp.bits >= 2 && sp.bits <= 8 && sp.bits != 7;
+  return sp.mode == MXFP4_M && sp.gs == 32 && sp.bits == 4 && dt == MLXQ_BFLOAT16;
+}
+
+// bfloat16 calls of 4/8-bit affine codes with K a multiple of 64 have the
+// prefill tile kernel, which rounds the dequantized weights to bfloat16, as
+// the strip kernel's only rival past 16 rows; other K ran on the skinny MFMA
+// kernel, which does not round them, and stays there.
+bool rounds_weights(const QmmSpec& sp) { return sp.mode != AFFINE || sp.K % 64 == 0; }
+
+// Dense calls (2-D weights) on the strip kernel.  MI355X, graph-timed:
+// - codes of 2, 3, 5 and 6 bits from 5 rows on, where the general tile kernel
+//   was the only other one (1-4 rows run the general decode kernel, whose
+//   weights are not rounded): 14336 x 4096 3-bit 8 rows 14.6 us vs 62.6, 64
+//   rows 23 vs 75; up to 128 rows;
+// - 4- and 8-bit codes and mxfp4 at 17-64 rows (fewer run the decode kernels,
+//   whose weights are not rounded): 14336 x 4096 4-bit 32 rows 18.9 vs 31.2
+//   on the prefill tiles, 64 rows 23 vs 33; 4096 x 4096 32 rows 10.5 vs 18.4;
+// - 65-128 rows of those where every wave multiplies at most 4 windows
+//   (short K, or few enough weight rows for a K split): 4096 x 4096 20.4 vs
+//   22.7, 1024 x 4096 13.9 vs 16.8; 14336 x 4096 (16 windows) 42 vs 37 stays
+//   on the tiles.
+bool try_strip(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, const mlxq_array* scales,
+               const mlxq_array* biases, mlxq_array* out, int64_t rows, hipStream_t stream, const ScratchSrc& ss) {
+  const Knobs& kn = knobs();
+  if (kn.strip == 0 || rows < 1 || !strip_types(sp, x, scales, biases)) return false;
+  const bool forced = kn.strip == 2;
+  const bool odd = sp.mode == AFFINE && sp.bits != 4 && sp.bits != 8;
+  if (!forced) {
+    // kernels forced by other switches stay forced
+    if (!kn.qmv_kernel.empty() || kn.qmm_tile >= 0 || kn.qmm_ksplit > 0 || kn.gen_ks > 0 || kn.qmm_min_rows != kQmmMinRows)
+      return false;
+    if (rows < (odd ? 5 : 17) || rows > 128) return false;
+    if (sp.out_dtype == MLXQ_BFLOAT16 && !odd && !rounds_weights(sp)) return false;
+  }
+  const int dev = current_device();
+  const int cus = device_info(dev).cus;
+  const int fmt = sp.mode == MXFP4_M ? mlxq::MXFP4 : mlxq::AFF4;
+  mlxq::StripPlan p = mlxq::strip_plan(fmt, sp.bits, sp.gs, rows, sp.N, sp.K, 0, cus, kn.strip_nwn, kn.strip_mt, kn.strip_ks);
+  if (!p.ok || (!forced && !odd && rows > 64 && p.windows > 4)) return false;
+  auto part = [&] { return (size_t)p.ks * rows * sp.N * sizeof(float); };
+  if (p.ks > 1 && !scratch_fits(dev, stream, part(), ss)) {
+    p = mlxq::strip_plan(fmt, sp.bits, sp.gs, rows, sp.N, sp.K, 0, cus, 0, 0, 1);  // no K ranges, no scratch
+    if (!p.ok) return false;
+  }
+  mlxq::StripArgs a{};
+  a.x = static_cast<const uint16_t*>(x->data);
+  a.w = static_cast<const uint32_t*>(w->data);
+  a.scales = scales->data;
+  a.biases = biases ? biases->data : nullptr;
+  a.out = static_cast<uint16_t*>(out->data);
+  a.xt = sp.out_dtype == MLXQ_FLOAT16 ? 1 : 0;
+  a.M = (int)rows;
+  a.N = (int)sp.N;
+  a.K = (int)sp.K;
+  a.gs_shift = gs_shift_of(sp.gs);
+  if (p.ks > 1) a.ws = reinterpret_cast<float*>(workspace(dev, stream, part(), ss));
+  hip_check(mlxq::strip_launch(fmt, sp.bits, a, p, stream), "qmm_strip launch");
+  if (p.ks > 1)
+    hip_check(mlxq::launch_splitk_reduce(a.ws, a.out, rows * sp.N, p.ks, stream, a.xt), "reduce launch");
+  return true;
+}
+
 // Route of a dense (2-D weight) bfloat16 call of `rows` activation rows on
 // the mid-size decode kernels, or DR_OTHER (row streaming, block MFMA,
 // prefill GEMM):
@@ -1390,12 +1485,6 @@ DenseRoute dense_route(const QmmSpec& sp, int64_t rows, int cus, bool single = t
   r.mid = mlxq::qmv_mid_plan(fmt, sp.gs, sp.N, sp.K, (int)rows, cus, knobs().mid_win);
   if (r.mid.ok) r.kind = DR_MID;
   return r;
-}
-
-int gs_shift_of(int gs) {
-  int shift = 0;
-  while ((1 << shift) < gs) shift++;
-  return shift;
 }
 
 mlxq::QmvMrArgs mr_args(const QmmSpec& sp, const uint16_t* x, int64_t rows, const uint32_t* w, const void* scales,
@@ -1582,6 +1671,7 @@ void run_quantized_matmul(const QmmSpec& sp, const mlxq_array* x, const mlxq_arr
       return;
     }
   }
+  if (View{w}.ndim() == 2 && try_strip(sp, x, w, scales, biases, out, rows_total, stream, ss)) return;
   if (!sp.fast) {
     View wv{w};
     const bool dense = wv.ndim() == 2 && sp.small_w;  // the float16 routes use buffer resources too

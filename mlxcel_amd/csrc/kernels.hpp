@@ -338,6 +338,39 @@ struct QmmGroupPlan {
 QmmGroupPlan qmm_group_plan(int fmt, int64_t N, int64_t K, int64_t E, int64_t B, int cus, int tiles_req = 0);
 hipError_t qmm_group_launch(const QmmGroupArgs& a, const QmmGroupPlan& p, hipStream_t stream);
 
+// Strip kernel (qmm_strip.hip): weights dequantized in registers into MFMA
+// operands; a few to ~100 activation rows per pass over a weight matrix.
+struct StripArgs {
+  const uint16_t* x;       // [M][K], bfloat16 (xt 0) or float16 (xt 1)
+  const uint32_t* w;       // packed codes [E][N][K*bits/32]
+  const void* scales;      // [E][N][K/gs] of x's type, or e8m0 (mxfp4)
+  const void* biases;      // like scales (affine)
+  uint16_t* out;           // [M][N]
+  float* ws;               // fp32 partials [ks][M][N] (ks > 1)
+  const uint32_t* rhs;     // sorted gathers: expert per row of x (32- or 64-bit, low word); null: dense
+  int rhs_stride;          // 32-bit words per index (1 or 2)
+  int M, N, K, gs_shift;
+  int xt;                  // 16-bit type: 0 bfloat16, 1 float16
+  int E;                   // experts (gathers)
+  int64_t w_expert_stride; // words per expert
+  int64_t s_expert_stride; // scales per expert
+  int ks, k_per_split;     // K ranges (dense), set by strip_launch
+};
+// 128-position windows per wave and staged step (LDS holds two steps of
+// activations; longer steps mean fewer barriers)
+constexpr int strip_wps(int mt, int nwn) { return mt == 1 && nwn >= 2 ? 2 : 1; }
+struct StripPlan {
+  bool ok = false;
+  int mt = 1;              // 16-row activation tiles per pass
+  int nwn = 4;             // waves along the weight rows (16 rows each)
+  int row_blocks = 0, ks = 1, k_per_split = 0;
+  int windows = 0;         // 128-position windows each wave multiplies
+  size_t lds = 0;
+};
+StripPlan strip_plan(int fmt, int bits, int gs, int64_t rows, int64_t N, int64_t K, int64_t experts, int cus,
+                     int nwn_req, int mt_req, int ks_req);
+hipError_t strip_launch(int fmt, int bits, const StripArgs& a, const StripPlan& p, hipStream_t stream);
+
 // Full-row decode kernel (qmv_fr.hip) for 1 or 2 activation rows per weight
 // matrix: 8 waves per workgroup, R whole rows per wave, activations staged in
 // LDS once per workgroup.

@@ -1,0 +1,88 @@
+// qmm_strip.hip — plan and launch of the strip kernel (qmm_strip.hpp), and
+// its bfloat16 instantiations for 4/8-bit affine codes and mxfp4.
+#include <algorithm>
+
+#include "qmm_strip.hpp"
+
+namespace mlxq {
+
+namespace {
+
+size_t strip_lds(int mt, int nwn, int gs) {
+  const int sr = (8 / nwn) * 128 * strip_wps(mt, nwn);
+  return (size_t)2 * mt * 16 * sr * 2 + (size_t)2 * (sr / gs) * (16 * nwn + 16) * 4 + 16;
+}
+
+// Microseconds of a launch on MI355X: start + per-window time of a wave
+// (fitted to graph-timed 4-bit g64 calls over 11 shapes from 1024 x 4096 to
+// 28672 x 4096; 3- and 6-bit codes lie within 15%), [log2(mt)][log2(nwn)].
+constexpr float kStart[4][3] = {{4.0f, 5.0f, 3.6f}, {4.7f, 4.1f, 3.2f}, {0.f, 4.9f, 3.9f}, {0.f, 0.f, 4.2f}};
+constexpr float kWindow[4][3] = {{1.0f, 0.65f, 0.70f}, {1.3f, 1.1f, 0.98f}, {0.f, 1.53f, 1.21f}, {0.f, 0.f, 2.4f}};
+
+}  // namespace
+
+StripPlan strip_plan(int fmt, int bits, int gs, int64_t rows, int64_t N, int64_t K, int64_t experts, int cus,
+                     int nwn_req, int mt_req, int ks_req) {
+  StripPlan p;
+  if (rows < 1 || N < 1 || K < 32 || K % 32 != 0 || K % gs != 0 || (fmt == MXFP4 && gs != 32)) return p;
+  if (rows * K * 2 >= ((int64_t)1 << 31) || N * (K / 32) * bits * 4 >= ((int64_t)1 << 31) || N * (K / gs) * 2 >= ((int64_t)1 << 31))
+    return p;
+  const int64_t per = experts > 0 ? (rows + experts - 1) / experts : rows;
+  int lm = per <= 16 ? 0 : per <= 32 ? 1 : per <= 64 ? 2 : 3;
+  // an expert's rows spread around the average and are taken 16 mt at a
+  // time: 32 at a time measured fastest from 12 to ~100 rows per expert (128
+  // experts of 768 x 2048, 64 rows each: 117 us vs 135 with 64 at a time),
+  // 128 past that (8 experts of 4096 x 2048, 256 rows each: 114 vs 127)
+  if (experts > 0) lm = per <= 11 ? 0 : per <= 100 ? 1 : 3;
+  for (int i = 0; i < 4; i++)
+    if (mt_req == 1 << i) lm = i;
+  const int mt = 1 << lm;
+  const int64_t passes = experts > 0 ? 1 : (rows + 16 * mt - 1) / (16 * mt);
+  float best = 0.f;
+  for (int ln = 0; ln < 3; ln++) {
+    const int nwn = 1 << ln;
+    if (kWindow[lm][ln] == 0.f || (nwn_req > 0 && nwn != nwn_req)) continue;
+    const int wps = strip_wps(mt, nwn), sr = (8 / nwn) * 128 * wps;
+    if (sr < 2 * gs || strip_lds(mt, nwn, gs) > kQmvLdsMax) continue;
+    const int64_t blocks = (N + 16 * nwn - 1) / (16 * nwn);
+    const int64_t steps = (K + sr - 1) / sr;
+    const int64_t ks_max = experts > 0 ? 1 : ks_req > 0 ? ks_req : std::min<int64_t>(16, std::max<int64_t>(1, cus / blocks));
+    for (int64_t ks = ks_req > 0 && experts <= 0 ? ks_req : 1; ks <= ks_max; ks++) {
+      const int64_t per_split = (steps + ks - 1) / ks;
+      const int64_t ksr = (steps + per_split - 1) / per_split;
+      const float windows = (float)((per_split + 1) / 2 * 2 * wps) * passes;  // steps run in pairs
+      const float rounds = std::max(1.f, (float)(blocks * ksr * std::max<int64_t>(experts, 1)) / cus);
+      // a second launch adds the K ranges' partials
+      const float reduce = ksr > 1 ? 2.5f + (float)(ksr * rows * N) * 8.f / 4e6f : 0.f;
+      const float us = kStart[lm][ln] + kWindow[lm][ln] * windows * rounds + reduce;
+      if (p.ok && us >= best) continue;
+      best = us;
+      p.ok = true;
+      p.mt = mt;
+      p.nwn = nwn;
+      p.row_blocks = (int)blocks;
+      p.ks = (int)ksr;
+      p.k_per_split = (int)std::min<int64_t>(per_split * sr, (int64_t)1 << 30);
+      p.windows = (int)windows;
+      p.lds = strip_lds(mt, nwn, gs);
+    }
+  }
+  if (p.ok && (p.row_blocks * (int64_t)16 * p.nwn >= ((int64_t)1 << 31) || p.ks > 65535 || experts > 65535)) p.ok = false;
+  return p;
+}
+
+hipError_t strip_launch(int fmt, int bits, const StripArgs& a_in, const StripPlan& p, hipStream_t stream) {
+  if (!p.ok) return hipErrorInvalidValue;
+  StripArgs a = a_in;
+  a.ks = p.ks;
+  a.k_per_split = p.k_per_split;
+  const dim3 grid((unsigned)p.row_blocks, (unsigned)(a.rhs ? a.E : p.ks));
+  if (fmt == MXFP4) return a.xt == 0 ? strip_launch_fmt<MXFP4, 4, 0>(a, p, grid, stream) : hipErrorInvalidValue;
+  if (bits == 4 || bits == 8) {
+    if (a.xt != 0) return strip_launch_f16(bits, a, p, grid, stream);
+    return bits == 4 ? strip_launch_fmt<AFF4, 4, 0>(a, p, grid, stream) : strip_launch_fmt<AFF4, 8, 0>(a, p, grid, stream);
+  }
+  return a.xt != 0 ? strip_launch_f16_odd(bits, a, p, grid, stream) : strip_launch_odd(bits, a, p, grid, stream);
+}
+
+}  // namespace mlxq

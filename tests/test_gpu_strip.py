@@ -1,0 +1,119 @@
+"""GPU parity of the strip kernel (qmm_strip.hpp): weights dequantized in
+registers into MFMA operands, 5-128 dense rows and expert-sorted gathers of
+affine codes, against the float64 numpy restatement of MLX's CPU kernels
+(oracle/generic.py).
+
+The sizes sit at the kernel's edges: the 16-row activation tiles (16/17,
+32/33, 64/65, 128), the 16-64-row weight blocks, the 128-position windows and
+the steps of several of them (K below one window, one past it, an odd number
+of groups), K ranges with their partial sums.  Tolerance: max|y - y_ref| /
+max|y_ref| <= 1e-2, the bound of every 16-bit result here (weights rounded to
+the 16-bit type, one rounding of the result).
+"""
+import numpy as np
+import pytest
+import torch
+
+import mlxcel_amd as mq
+from oracle import generic as og
+from helpers import announce, dev_u32, setknob
+
+pytestmark = pytest.mark.gpu
+
+TD = {"bfloat16": torch.bfloat16, "float16": torch.float16}
+
+
+def _dev(vals, dt):
+    t = torch.from_numpy(np.asarray(vals, dtype=np.float32)).to(TD[dt]).cuda()
+    return t, t.float().cpu().numpy().astype(np.float64)
+
+
+def _weights(rng, shape, K, bits, gs, dt):
+    wqn = og.pack_codes(rng.integers(0, 1 << bits, size=shape + (K,)), bits)
+    s, sv = _dev(rng.uniform(0.002, 0.02, size=shape + (K // gs,)), dt)
+    b, bv = _dev(rng.uniform(-0.1, 0.1, size=shape + (K // gs,)), dt)
+    return (dev_u32(wqn), s, b), (wqn, sv, bv)
+
+
+def _rel(y, want, dt):
+    got = y.float().cpu().numpy().astype(np.float64)
+    want = og.round_to(want, dt)
+    return float(np.abs(got - want).max() / max(np.abs(want).max(), 1e-30))
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, 5, 6, 8])
+@pytest.mark.parametrize("dt", ["bfloat16", "float16"])
+@pytest.mark.parametrize("M,N,K,gs,nwn,ks", [
+    (5, 33, 32, 32, 4, 1), (16, 64, 160, 32, 2, 1), (16, 17, 1056, 32, 1, 2), (17, 65, 4096, 128, 4, 3),
+    (32, 1, 192, 64, 1, 1), (33, 130, 2112, 64, 2, 2), (64, 100, 640, 128, 4, 1), (65, 48, 1088, 64, 4, 2),
+    (128, 70, 576, 64, 4, 1), (300, 40, 256, 32, 4, 1)])
+def test_dense_edges(monkeypatch, bits, dt, M, N, K, gs, nwn, ks):
+    setknob(monkeypatch, "MLXQ_STRIP", "2")
+    setknob(monkeypatch, "MLXQ_STRIP_NWN", str(nwn))
+    setknob(monkeypatch, "MLXQ_STRIP_KS", str(ks))
+    rng = np.random.default_rng(41000 + 100 * bits + M)
+    announce("strip", bits, dt, M, N, K, gs, nwn, ks)
+    x, xv = _dev(rng.standard_normal((M, K)), dt)
+    (wq, s, b), (wqn, sv, bv) = _weights(rng, (N,), K, bits, gs, dt)
+    y = mq.quantized_matmul(x, wq, s, b, True, gs, bits)
+    assert _rel(y, og.qmm(xv, wqn, sv, bv, True, gs, bits), dt) <= 1e-2
+
+
+@pytest.mark.parametrize("bits,M", [(3, 5), (6, 128), (4, 17), (8, 64), (4, 100)])
+def test_default_route_matches_other_kernels(monkeypatch, bits, M):
+    rng = np.random.default_rng(42000 + bits)
+    N, K, gs = 513, 4096, 64
+    announce("strip default", bits, M)
+    x, xv = _dev(rng.standard_normal((M, K)), "bfloat16")
+    (wq, s, b), (wqn, sv, bv) = _weights(rng, (N,), K, bits, gs, "bfloat16")
+    y = mq.quantized_matmul(x, wq, s, b, True, gs, bits)
+    again = mq.quantized_matmul(x, wq, s, b, True, gs, bits)
+    setknob(monkeypatch, "MLXQ_STRIP", "0")
+    other = mq.quantized_matmul(x, wq, s, b, True, gs, bits)
+    want = og.qmm(xv, wqn, sv, bv, True, gs, bits)
+    assert torch.equal(y, again)
+    assert _rel(y, want, "bfloat16") <= 1e-2 and _rel(other, want, "bfloat16") <= 1e-2
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), 3e38, 2.0 ** 101])
+def test_extreme_scales_stay_in_their_row(monkeypatch, value):
+    # scales past 2^100 take the slower conversion; a row's NaN or infinity
+    # must not reach its neighbours through the positions past K
+    setknob(monkeypatch, "MLXQ_STRIP", "2")
+    rng = np.random.default_rng(43000)
+    M, N, K, gs, bits = 9, 40, 96, 32, 4
+    announce("strip extreme scales", value)
+    x, xv = _dev(rng.standard_normal((M, K)), "bfloat16")
+    (wq, s, b), (wqn, sv, bv) = _weights(rng, (N,), K, bits, gs, "bfloat16")
+    s[5] = value
+    y = mq.quantized_matmul(x, wq, s, b, True, gs, bits).float().cpu().numpy().astype(np.float64)
+    setknob(monkeypatch, "MLXQ_STRIP", "0")
+    y0 = mq.quantized_matmul(x, wq, s, b, True, gs, bits).float().cpu().numpy().astype(np.float64)
+    want = og.round_to(og.qmm(xv, wqn, sv, bv, True, gs, bits), "bfloat16")
+    rest = [n for n in range(N) if n != 5]
+    assert np.abs(y[:, rest] - want[:, rest]).max() <= 1e-2 * np.abs(want[:, rest]).max()
+    if value == 2.0 ** 101:  # finite sums: the other kernel's values up to the summation order
+        assert np.abs(y[:, 5] - y0[:, 5]).max() <= 1e-2 * np.abs(y0[:, 5]).max()
+    elif value == value and value < 1e39:
+        assert np.isfinite(y[:, rest]).all()
+    else:
+        assert np.isnan(y[:, 5]).all()
+
+
+def test_mxfp4_special_scales(monkeypatch):
+    setknob(monkeypatch, "MLXQ_STRIP", "2")
+    rng = np.random.default_rng(44000)
+    M, N, K = 18, 37, 224
+    announce("strip mxfp4 scales")
+    x, xv = _dev(rng.standard_normal((M, K)), "bfloat16")
+    wqn = og.pack_codes(rng.integers(0, 16, size=(N, K)), 4)
+    sc = rng.integers(120, 130, size=(N, K // 32)).astype(np.uint8)
+    sc[3], sc[4], sc[7, 0] = 0, 230, 255  # 2^-127, 2^103 (254 would overflow the sums), NaN
+    y = mq.quantized_matmul(x, dev_u32(wqn), torch.from_numpy(sc).cuda(), None, True, 32, 4, "mxfp4")
+    got = y.float().cpu().numpy().astype(np.float64)
+    want = og.round_to(og.qmm(xv, wqn, sc, None, True, 32, 4, "mxfp4"), "bfloat16")
+    assert np.isnan(got[:, 7]).all()
+    for n in range(N):
+        if n != 7:
+            ok = np.isclose(got[:, n], want[:, n], rtol=1e-2, atol=1e-2 * np.nanmax(np.abs(want[:, n])))
+            assert ok.all(), n
