@@ -1390,6 +1390,51 @@ bool try_strip(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, cons
   return true;
 }
 
+// Sorted gathers of affine codes with one row per entry and at least 8
+// entries per touched expert, where the kernels for grouped rows round the
+// weights too (fewer run the block-MFMA search kernel, which does not): a
+// workgroup per 64 weight rows of an expert finds the expert's entries in
+// the indices itself.  MI355X, 128 experts of 768 x 2048 4-bit, top 8,
+// against grouping on the device + 16x16-MFMA tiles: 128 tokens 41 us vs
+// 104, 512 tokens 79 vs 119, 1024 tokens 117 vs 180; 8 experts of 4096 x
+// 2048 8-bit, top 2: 64 tokens 20 vs 65, 1024 tokens 114 vs 211.
+bool try_strip_gather(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, const mlxq_array* scales,
+                      const mlxq_array* biases, const DirectIdx& dl, const DirectIdx& dr, mlxq_array* out, int64_t B,
+                      int64_t E, hipStream_t stream) {
+  const Knobs& kn = knobs();
+  if (kn.strip == 0 || !strip_types(sp, x, scales, biases)) return false;
+  if (kn.strip != 2 && (sp.mode != AFFINE || !rounds_weights(sp) || kn.gather_group >= 0 || kn.gather_sorted == 0 || B < 8 * std::min(E, B)))
+    return false;
+  // one row of x per entry, indices read in place
+  if (!dr.ok || !dr.p || !dl.ok || dl.p || dl.div != 1) return false;
+  const int fmt = sp.mode == MXFP4_M ? mlxq::MXFP4 : mlxq::AFF4;
+  const mlxq::StripPlan p = mlxq::strip_plan(fmt, sp.bits, sp.gs, B, sp.N, sp.K, E, device_info(current_device()).cus,
+                                             kn.strip_nwn, kn.strip_mt, 0);
+  if (!p.ok) return false;
+  // many rows for few workgroups: the passes of 128 rows run one after the
+  // other (8 experts of 768 x 2048, 1024 rows each: 190 us vs 108 on the
+  // tiles; 8 of 2048 x 2048, 512 rows each, 256 workgroups: 81 vs 124)
+  if (kn.strip != 2 && B > 128 * E && p.row_blocks * E < device_info(current_device()).cus) return false;
+  mlxq::StripArgs a{};
+  a.x = static_cast<const uint16_t*>(x->data);
+  a.w = static_cast<const uint32_t*>(w->data);
+  a.scales = scales->data;
+  a.biases = biases ? biases->data : nullptr;
+  a.out = static_cast<uint16_t*>(out->data);
+  a.xt = sp.out_dtype == MLXQ_FLOAT16 ? 1 : 0;
+  a.M = (int)B;
+  a.N = (int)sp.N;
+  a.K = (int)sp.K;
+  a.gs_shift = gs_shift_of(sp.gs);
+  a.rhs = dr.p;
+  a.rhs_stride = dr.stride;
+  a.E = (int)E;
+  a.w_expert_stride = View{w}.dim(-2) * View{w}.dim(-1);
+  a.s_expert_stride = View{scales}.dim(-2) * View{scales}.dim(-1);
+  hip_check(mlxq::strip_launch(fmt, sp.bits, a, p, stream), "gather strip launch");
+  return true;
+}
+
 // Route of a dense (2-D weight) bfloat16 call of `rows` activation rows on
 // the mid-size decode kernels, or DR_OTHER (row streaming, block MFMA,
 // prefill GEMM):
@@ -1967,6 +2012,10 @@ void gather_run(GatherSpec& g, const mlxq_array* x, const mlxq_array* w, const m
       return;
     }
   }
+
+  if (sorted_indices && M == 1 && try_strip_gather(sp, x, w, scales, biases, direct_index(lhs_indices, dsh[0], g.idx_shape),
+                                                   direct_index(rhs_indices, dsh[1], g.idx_shape), out, B, E, stream))
+    return;
 
   // Many rows per expert (MoE prefill, large batches): group rows by expert
   // on the device, then one GEMM tile reads each expert's weights once per

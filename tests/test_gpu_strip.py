@@ -117,3 +117,18 @@ def test_mxfp4_special_scales(monkeypatch):
         if n != 7:
             ok = np.isclose(got[:, n], want[:, n], rtol=1e-2, atol=1e-2 * np.nanmax(np.abs(want[:, n])))
             assert ok.all(), n
+
+
+@pytest.mark.parametrize("bits,gs", [(4, 64), (8, 32), (4, 128)])
+@pytest.mark.parametrize("counts", [[8, 8, 8, 8], [0, 40, 1, 0, 33, 16], [0, 0, 130, 0, 300], [64, 0]])
+@pytest.mark.parametrize("idx", [torch.int32, torch.int64])
+def test_sorted_gather(bits, gs, counts, idx):
+    rng = np.random.default_rng(45000 + bits + sum(counts))
+    E, N, K = len(counts), 100, gs * 5
+    ids = np.repeat(np.arange(E), counts)
+    announce("strip gather", bits, gs, counts, idx)
+    x, xv = _dev(rng.standard_normal((len(ids), 1, K)), "bfloat16")
+    (wq, s, b), (wqn, sv, bv) = _weights(rng, (E, N), K, bits, gs, "bfloat16")
+    y = mq.gather_qmm(x, wq, s, b, None, torch.from_numpy(ids).to(idx).cuda(), True, gs, bits, "affine", True)
+    want = np.stack([og.qmm(xv[i], wqn[e], sv[e], bv[e], True, gs, bits) for i, e in enumerate(ids)])
+    assert _rel(y, want, "bfloat16") <= 1e-2
