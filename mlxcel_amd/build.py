@@ -46,6 +46,7 @@ SOURCES = {
     "qmv_mr.hip": [],
     "qmm_group.hip": [],
     "qmm.hip": [],
+    "qmm_odd.hip": [],
     "qmm_strip.hip": [],
     "qmm_strip_odd.hip": [],
     "qmm_strip_f16.hip": [],

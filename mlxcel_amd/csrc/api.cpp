@@ -527,6 +527,18 @@ void alloc_counters(Workspace& w, hipStream_t stream) {
   hip_check(hipMemsetAsync(w.data, 0, w.bytes, stream), "hipMemsetAsync (stream-K counters)");
 }
 
+// Whether a call may take `bytes` of scratch without allocating under a
+// capture (or past the fixed scratch).
+bool scratch_fits(int dev, hipStream_t stream, size_t bytes, const ScratchSrc& ss) {
+  if (ss.fixed) return bytes <= ss.max;
+  {
+    std::lock_guard<std::mutex> lk(g_mu);
+    const auto it = g_ws.find({dev, stream, 0});
+    if (it != g_ws.end() && it->second.bytes >= bytes) return true;
+  }
+  return !stream_capturing(stream);
+}
+
 // The prefill plan of a dense call: stream-K only where its partials and
 // counters can be had without allocating under a capture, and not for the
 // no-allocation entry point (its fixed scratch is small); otherwise the plan
@@ -537,6 +549,10 @@ mlxq::QmmPlan prefill_plan(int fmt, int gs, int64_t rows, int64_t N, int64_t K, 
   *cnt = nullptr;
   const int cus = device_info(dev).cus;
   mlxq::QmmPlan qp = mlxq::qmm_plan(fmt, gs, rows, N, K, cus, tile_req, ksplit_req, mix, ss.fixed ? 0 : streamk);
+  // a K split whose partials cannot be had here: the plan whose splits are
+  // powers of two (2-, 3-, 5- and 6-bit codes: the general kernel)
+  if (qp.ok && qp.ksplit > 1 && !scratch_fits(dev, stream, (size_t)qp.ksplit * rows * N * sizeof(float), ss))
+    qp = mlxq::qmm_plan(fmt, gs, rows, N, K, cus, tile_req, ksplit_req, mix, ss.fixed ? 0 : streamk, false);
   if (qp.sk_len <= 0) return qp;
   std::lock_guard<std::mutex> lk(g_mu);
   const bool capturing = stream_capturing(stream);
@@ -1267,13 +1283,28 @@ bool try_mid_f16(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, co
   return true;
 }
 
+// Operands of the strip kernel: transpose=true; x, scales and biases all
+// bfloat16 or all float16 with affine codes of 2-6 or 8 bits, or bfloat16 x
+// with mxfp4.
+bool strip_types(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* scales, const mlxq_array* biases) {
+  if (!sp.transpose || !sp.small_w) return false;
+  const int dt = sp.out_dtype;
+  if ((dt != MLXQ_BFLOAT16 && dt != MLXQ_FLOAT16) || x->dtype != dt) return false;
+  if (sp.mode == AFFINE)
+    return biases && scales->dtype == dt && biases->dtype == dt && sp.bits >= 2 && sp.bits <= 8 && sp.bits != 7;
+  return sp.mode == MXFP4_M && sp.gs == 32 && sp.bits == 4 && dt == MLXQ_BFLOAT16;
+}
+
 // float16 prefill (rows >= MLXQ_QMM_MIN_ROWS once the mid-size kernels have
 // declined): the 32x32-MFMA tile kernel's float16 instantiation; a requested
 // tile of the 16x16-MFMA kernel (bfloat16 only) falls back to the planner's.
-bool try_qmm_f16(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, const mlxq_array* scales,
-                 const mlxq_array* biases, mlxq_array* out, int64_t rows, hipStream_t stream, const ScratchSrc& ss) {
-  if (!f16_affine(sp, x, scales, biases) || rows < knobs().qmm_min_rows) return false;
-  const int fmt = fmt_of(sp.mode, sp.bits);
+bool try_qmm_tile(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, const mlxq_array* scales,
+                  const mlxq_array* biases, mlxq_array* out, int64_t rows, hipStream_t stream, const ScratchSrc& ss) {
+  const bool odd = sp.mode == AFFINE && sp.bits != 4 && sp.bits != 8;
+  if (odd ? (!strip_types(sp, x, scales, biases) || rows <= 128 || knobs().gen_ks > 0) : !f16_affine(sp, x, scales, biases))
+    return false;
+  if (rows < knobs().qmm_min_rows) return false;
+  const int fmt = odd ? mlxq::kAffOdd + sp.bits : fmt_of(sp.mode, sp.bits);
   const int dev = current_device();
   const int tile_req = knobs().qmm_tile >= 4 ? knobs().qmm_tile : -1;
   uint32_t* cnt = nullptr;
@@ -1295,7 +1326,7 @@ bool try_qmm_f16(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, co
   q.gs_shift = shift;
   q.ksplit = qp.ksplit;
   q.ksteps_per_split = qp.ksteps_per_split;
-  q.xt = 1;
+  q.xt = sp.out_dtype == MLXQ_FLOAT16 ? 1 : 0;
   if (qp.ksplit > 1)
     q.ws = reinterpret_cast<float*>(workspace(dev, stream, (size_t)qp.ksplit * rows * sp.N * sizeof(float), ss));
   if (qp.sk_len > 0) {
@@ -1305,30 +1336,6 @@ bool try_qmm_f16(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, co
   }
   hip_check(mlxq::qmm_launch(fmt, q, qp, stream), "qmm launch");
   return true;
-}
-
-// Whether a call may take `bytes` of scratch without allocating under a
-// capture (or past the fixed scratch).
-bool scratch_fits(int dev, hipStream_t stream, size_t bytes, const ScratchSrc& ss) {
-  if (ss.fixed) return bytes <= ss.max;
-  {
-    std::lock_guard<std::mutex> lk(g_mu);
-    const auto it = g_ws.find({dev, stream, 0});
-    if (it != g_ws.end() && it->second.bytes >= bytes) return true;
-  }
-  return !stream_capturing(stream);
-}
-
-// Operands of the strip kernel: transpose=true; x, scales and biases all
-// bfloat16 or all float16 with affine codes of 2-6 or 8 bits, or bfloat16 x
-// with mxfp4.
-bool strip_types(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* scales, const mlxq_array* biases) {
-  if (!sp.transpose || !sp.small_w) return false;
-  const int dt = sp.out_dtype;
-  if ((dt != MLXQ_BFLOAT16 && dt != MLXQ_FLOAT16) || x->dtype != dt) return false;
-  if (sp.mode == AFFINE)
-    return biases && scales->dtype == dt && biases->dtype == dt && sp.bits >= 2 && sp.bits <= 8 && sp.bits != 7;
-  return sp.mode == MXFP4_M && sp.gs == 32 && sp.bits == 4 && dt == MLXQ_BFLOAT16;
 }
 
 // bfloat16 calls of 4/8-bit affine codes with K a multiple of 64 have the
@@ -1368,10 +1375,8 @@ bool try_strip(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, cons
   mlxq::StripPlan p = mlxq::strip_plan(fmt, sp.bits, sp.gs, rows, sp.N, sp.K, 0, cus, kn.strip_nwn, kn.strip_mt, kn.strip_ks);
   if (!p.ok || (!forced && !odd && rows > 64 && p.windows > 4)) return false;
   auto part = [&] { return (size_t)p.ks * rows * sp.N * sizeof(float); };
-  if (p.ks > 1 && !scratch_fits(dev, stream, part(), ss)) {
-    p = mlxq::strip_plan(fmt, sp.bits, sp.gs, rows, sp.N, sp.K, 0, cus, 0, 0, 1);  // no K ranges, no scratch
-    if (!p.ok) return false;
-  }
+  // partials that cannot be had here: the kernels below
+  if (p.ks > 1 && !scratch_fits(dev, stream, part(), ss)) return false;
   mlxq::StripArgs a{};
   a.x = static_cast<const uint16_t*>(x->data);
   a.w = static_cast<const uint32_t*>(w->data);
@@ -1724,7 +1729,7 @@ void run_quantized_matmul(const QmmSpec& sp, const mlxq_array* x, const mlxq_arr
     if (dense && try_kq_f16(sp, x, w, scales, biases, out, rows_total, stream)) return;
     if (dense && try_rs_f16(sp, x, w, scales, biases, out, rows_total, stream)) return;
     if (dense && try_mid_f16(sp, x, w, scales, biases, out, rows_total, stream, ss)) return;
-    if (dense && try_qmm_f16(sp, x, w, scales, biases, out, rows_total, stream, ss)) return;
+    if (dense && try_qmm_tile(sp, x, w, scales, biases, out, rows_total, stream, ss)) return;
     if (wv.ndim() == 2) {
       // every leading dim of x folds into rows
       run_gen(sp, x, w, scales, biases, out, rows_total, 1, 1, 1, nullptr, stream, ss);

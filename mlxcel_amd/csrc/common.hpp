@@ -13,12 +13,16 @@
 namespace mlxq {
 
 enum Fmt : int { AFF4 = 0, AFF8 = 1, MXFP4 = 2 };
+// Format code of affine codes of any other width: kAffOdd + bits.
+constexpr int kAffOdd = 16;
+constexpr int fmt_bits(int fmt) { return fmt >= kAffOdd ? fmt - kAffOdd : fmt == AFF8 ? 8 : 4; }
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
 
 // ---- bf16 <-> f32 (bit exact; round to nearest even, NaN -> 0x7FC0, which is
 // MLX's `_MLX_BFloat16(float)`) ---------------------------------------------
@@ -283,6 +287,41 @@ __device__ __forceinline__ void sorted_run(const uint32_t* idx, int stride, int 
   end = res[1];
 }
 
+
+// ---- affine codes of any width ------------------------------------------------
+// 32 codes of BITS bits are BITS consecutive words of MLX's little-endian bit
+// stream; code i of them, zero-extended.
+template <int BITS>
+__device__ __forceinline__ uint32_t code_at(const uint32_t (&w)[BITS], int i) {
+  const int wd = (i * BITS) >> 5, sh = (i * BITS) & 31;
+  if (sh + BITS <= 32) return __builtin_amdgcn_ubfe(w[wd], sh, BITS);
+  return __builtin_amdgcn_ubfe(__builtin_amdgcn_alignbit(w[wd + 1 < BITS ? wd + 1 : wd], w[wd], sh), 0, BITS);
+}
+
+template <int BITS>
+__device__ __forceinline__ void load_codes(const __amdgpu_buffer_rsrc_t& r, uint32_t o, int so, uint32_t (&w)[BITS]) {
+  int p = 0;
+  if constexpr (BITS >= 4) {
+#pragma unroll
+    for (int c = 0; c < BITS / 4; c++) {
+      const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, o + 16u * c, so, 0));
+#pragma unroll
+      for (int e = 0; e < 4; e++) w[4 * c + e] = v[e];
+    }
+    p = BITS / 4 * 4;
+  }
+  if constexpr (BITS % 4 == 3) {
+    const u32x3 v = __builtin_bit_cast(u32x3, __builtin_amdgcn_raw_buffer_load_b96(r, o + 4u * p, so, 0));
+#pragma unroll
+    for (int e = 0; e < 3; e++) w[p + e] = v[e];
+  } else if constexpr (BITS % 4 == 2) {
+    const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, o + 4u * p, so, 0));
+    w[p] = v[0];
+    w[p + 1] = v[1];
+  } else if constexpr (BITS % 4 == 1) {
+    w[p] = __builtin_amdgcn_raw_buffer_load_b32(r, o + 4u * p, so, 0);
+  }
+}
 
 // c + a.lo * b.lo + a.hi * b.hi over bf16 pairs, fp32 accumulate
 __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {

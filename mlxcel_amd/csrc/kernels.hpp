@@ -454,8 +454,10 @@ QmmPlan qmm_plan_grouped(int fmt, int gs, int64_t N, int64_t K, int tile);
 // tile_req / ksplit_req < 0 (or 0 for ksplit) choose by shape.
 // mix: allow the two-launch plan (tile2) when neither tile nor split is requested;
 // streamk: allow the stream-K plan there (it takes precedence).
+// fit_round: allow tiles and K splits that fill one round of the CUs
+// (false: splits by powers of two, and no plan for 2/3/5/6-bit codes).
 QmmPlan qmm_plan(int fmt, int gs, int64_t M, int64_t N, int64_t K, int num_cus, int tile_req, int ksplit_req,
-                 int mix = 1, int streamk = 0);
+                 int mix = 1, int streamk = 0, bool fit_round = true);
 hipError_t qmm_launch(int fmt, const QmmArgs& a, const QmmPlan& p, hipStream_t stream);
 // out[i] = bf16(sum over z < ks of ws[z * n + i]) (qmv.hip)
 // out (16-bit type xt: 0 bfloat16, 1 float16) = sum over ks fp32 partials, in split order

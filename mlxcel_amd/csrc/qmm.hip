@@ -21,6 +21,9 @@
 // When the grid would leave CUs idle (short M), K is split across
 // workgroups and the fp32 partials are summed by a second kernel in a fixed
 // order (bitwise reproducible).
+#include <algorithm>
+#include <cmath>
+
 #include "qmm_tile.hpp"
 
 namespace mlxq {
@@ -242,17 +245,67 @@ bool is_tile_kernel(int tile) { return tile >= 4; }
 
 int qmm_tile_rows(int tile) { return tile >= 0 && tile < kTiles ? kBM[tile] : 0; }
 
+namespace {
+// Tile and K split of a grid that fits about one round of the CUs (129-1024
+// rows; the 2-, 3-, 5- and 6-bit codes, which have no 256 x 128 tile on 8
+// waves, at any row count).  One round of 256 x 128 tiles (3/4 to all of the
+// CUs) runs unsplit, else 0.58 to one round of 256 x 256 tiles does (14336 x
+// 4096: 512 rows 76 us, 768 rows 107).  Otherwise each tile with no split,
+// the split that fills the round and one less is priced as
+//   start + K-steps per workgroup * (c1 + c2 * fill) + partial sums
+// fitted to 300 graph-timed calls on MI355X (4- and 8-bit codes, seven
+// shapes, 129-1024 rows, 9% rms); over those the choice is within 1.3% of
+// the fastest (tile, split) on average, where splits by powers of two alone
+// were 10% off: 1900 x 1152 256 rows 16.2 us vs 20.5, 6144 x 4096 333 rows
+// 41.5 vs 47, 768 rows 62 vs 73, 4096 x 14336 768 rows 111 vs 134.
+int plan_mid(bool odd, int64_t M, int64_t N, int nks, int num_cus, int& ks_out) {
+  struct Cost {
+    int tile, slots, min_steps;  // workgroups per CU, K-steps a split keeps
+    float start, c1, c2;
+  };
+  constexpr Cost costs[3] = {{4, 1, 8, 14.7f, 1.474f, 0.10f}, {6, 2, 4, 9.6f, 0.583f, 0.677f}, {8, 1, 8, 10.4f, 0.831f, 0.286f}};
+  auto tiles_of = [&](int t) { return ((M + kBM[t] - 1) / kBM[t]) * ((N + kBN[t] - 1) / kBN[t]); };
+  ks_out = 1;
+  if (!odd && tiles_of(8) * 4 >= (int64_t)num_cus * 3 && tiles_of(8) <= num_cus) return 8;
+  if (tiles_of(4) * 100 >= (int64_t)num_cus * 58 && tiles_of(4) <= num_cus) return 4;
+  int best_tile = 6;
+  float best = 0.f;
+  for (const Cost& c : costs) {
+    if (odd && c.tile == 8) continue;
+    const int64_t tiles = tiles_of(c.tile), slots = (int64_t)c.slots * num_cus;
+    const int mx = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(slots / tiles, nks / c.min_steps), 16));
+    for (int ks : {1, mx - 1, mx}) {
+      if (ks < 1) continue;
+      const int steps = (nks + ks - 1) / ks, ksr = (nks + steps - 1) / steps;
+      const float x = (float)(tiles * ksr) / slots;
+      const float per = x <= 1.f ? c.c1 + c.c2 * x : (c.c1 + c.c2) * 0.5f * (std::ceil(x) + x);
+      const float us = c.start + per * steps + (ksr > 1 ? 2.5f + (float)ksr * M * N * 1e-6f : 0.f);
+      if (best > 0.f && us >= best) continue;
+      best = us;
+      best_tile = c.tile;
+      ks_out = ksr;
+    }
+  }
+  return best_tile;
+}
+}  // namespace
+
 QmmPlan qmm_plan(int fmt, int gs, int64_t M, int64_t N, int64_t K, int num_cus, int tile_req, int ksplit_req,
-                 int mix, int streamk) {
+                 int mix, int streamk, bool fit_round) {
   QmmPlan p;
-  const int bits = fmt == AFF8 ? 8 : 4;
+  if (fmt >= kAffOdd && !fit_round) return p;
+  const int bits = fmt_bits(fmt);
+  const bool odd = fmt >= kAffOdd;  // tiles 4 and 6 only
+  if (odd && tile_req != 4 && tile_req != 6) tile_req = -1;
   if (K % BK != 0 || K % gs != 0 || M <= 0 || N <= 0) return p;
   if (M * K * 2 >= ((int64_t)1 << 31) || N * K * bits / 8 >= ((int64_t)1 << 31)) return p;
   const int nks = (int)(K / BK);
   auto tiles_of = [&](int t) { return ((M + kBM[t] - 1) / kBM[t]) * ((N + kBN[t] - 1) / kBN[t]); };
-  int tile;
+  int tile, ks_planned = 0;
   if (tile_req >= 0 && tile_req < kTiles) {
     tile = tile_req;
+  } else if (fit_round && odd) {
+    tile = plan_mid(odd, M, N, nks, num_cus, ks_planned);
   } else {
     // 256 x 256 (8 waves) when there are enough tiles or K is long enough
     // for a K split to fill the CUs; else 128 x 128, two workgroups per CU.
@@ -279,6 +332,8 @@ QmmPlan qmm_plan(int fmt, int gs, int64_t M, int64_t N, int64_t K, int num_cus, 
   int ks = 1;
   if (ksplit_req > 0) {
     ks = ksplit_req;
+  } else if (ks_planned > 0) {
+    ks = ks_planned;
   } else {
     // split K while the grid covers less than the CUs (up to two workgroups
     // per CU for few rows, where each tile is cheap) and each split keeps >= 8
@@ -313,7 +368,7 @@ QmmPlan qmm_plan(int fmt, int gs, int64_t M, int64_t N, int64_t K, int num_cus, 
   // time, which costs ~30% per step (MI355X, K=4096, 4-bit: 12288 x 1536
   // rows, 1.125 rounds, 170.5 us vs 196.6 on the two-launch plan; 14336 x
   // 2048 rows, 1.75 rounds, 269 vs 233).  streamk > 1 forces that run length.
-  if (streamk && tile_req < 0 && ksplit_req <= 0 && p.tile == 4 && p.ksplit == 1 && tiles > num_cus &&
+  if (streamk && !odd && tile_req < 0 && ksplit_req <= 0 && p.tile == 4 && p.ksplit == 1 && tiles > num_cus &&
       fmt != MXFP4 && (streamk > 1 || (tiles < 2 * (int64_t)num_cus && (tiles - num_cus) * 8 <= num_cus))) {
     const int64_t steps = tiles * nks;
     const int64_t len = streamk > 1 ? streamk : (steps + num_cus - 1) / num_cus;
@@ -323,7 +378,7 @@ QmmPlan qmm_plan(int fmt, int gs, int64_t M, int64_t N, int64_t K, int num_cus, 
       return p;
     }
   }
-  if (mix && tile_req < 0 && ksplit_req <= 0 && p.tile == 4 && p.ksplit == 1 && tiles > num_cus) {
+  if (mix && !odd && tile_req < 0 && ksplit_req <= 0 && p.tile == 4 && p.ksplit == 1 && tiles > num_cus) {
     const int64_t nb = (tiles / num_cus) * num_cus / p.tiles_m;  // 256-wide column tiles in whole rounds
     const int64_t n1 = nb * kBN[4];
     const int64_t tn2 = (N - n1 + kBN[8] - 1) / kBN[8];
@@ -433,7 +488,10 @@ hipError_t qmm_launch(int fmt, const QmmArgs& a_in, const QmmPlan& p, hipStream_
   a.tiles_n = p.tiles_n;
   a.m_fast = p.m_fast;
   if (p.sk_len <= 0) a.sk_len = 0;
-  switch (fmt) {
+  if (fmt >= kAffOdd) {
+    if ((p.tile != 4 && p.tile != 6) || p.tile2 >= 0 || p.sk_len > 0 || a.seg) return hipErrorInvalidValue;
+    qmm_launch_odd(fmt - kAffOdd, a, p.tile, p.ksplit, stream);
+  } else switch (fmt) {
     case AFF4: qmm_launch_fmt<AFF4>(a, p, stream); break;
     case AFF8: qmm_launch_fmt<AFF8>(a, p, stream); break;
     default: qmm_launch_fmt<MXFP4>(a, p, stream); break;

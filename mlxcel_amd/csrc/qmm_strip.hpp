@@ -48,48 +48,12 @@ namespace mlxq {
 typedef float sf32x2 __attribute__((ext_vector_type(2)));
 constexpr uint32_t kBigScale = (127u + 100u) << 7;  // exponent field of a bfloat16 2^100
 
-typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
-
 template <int XT>
 __device__ __forceinline__ uint32_t strip_pack(float lo, float hi) {
   if constexpr (XT == 0) return __builtin_bit_cast(uint32_t, __builtin_convertvector(sf32x2{lo, hi}, bf16x2));
   else {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(sf32x2{lo, hi}, h2));
-  }
-}
-
-// Code i of a lane's 32 (BITS consecutive words of the little-endian bit
-// stream).
-template <int BITS>
-__device__ __forceinline__ uint32_t strip_code(const uint32_t (&w)[BITS], int i) {
-  const int wd = (i * BITS) >> 5, sh = (i * BITS) & 31;
-  if (sh + BITS <= 32) return __builtin_amdgcn_ubfe(w[wd], sh, BITS);
-  return __builtin_amdgcn_ubfe(__builtin_amdgcn_alignbit(w[wd + 1 < BITS ? wd + 1 : wd], w[wd], sh), 0, BITS);
-}
-
-template <int BITS>
-__device__ __forceinline__ void strip_load(const __amdgpu_buffer_rsrc_t& r, uint32_t o, int so, uint32_t (&w)[BITS]) {
-  int p = 0;
-  if constexpr (BITS >= 4) {
-#pragma unroll
-    for (int c = 0; c < BITS / 4; c++) {
-      const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, o + 16u * c, so, 0));
-#pragma unroll
-      for (int e = 0; e < 4; e++) w[4 * c + e] = v[e];
-    }
-    p = BITS / 4 * 4;
-  }
-  if constexpr (BITS % 4 == 3) {
-    const u32x3 v = __builtin_bit_cast(u32x3, __builtin_amdgcn_raw_buffer_load_b96(r, o + 4u * p, so, 0));
-#pragma unroll
-    for (int e = 0; e < 3; e++) w[p + e] = v[e];
-  } else if constexpr (BITS % 4 == 2) {
-    const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, o + 4u * p, so, 0));
-    w[p] = v[0];
-    w[p + 1] = v[1];
-  } else if constexpr (BITS % 4 == 1) {
-    w[p] = __builtin_amdgcn_raw_buffer_load_b32(r, o + 4u * p, so, 0);
   }
 }
 
@@ -164,7 +128,7 @@ __global__ __launch_bounds__(512, 2) void qmm_strip_kernel(const StripArgs a) {
   uint32_t wv[RD][BITS];
   auto load_window = [&](int slot, int step, int w) {
     const bool live = step < nsteps;
-    strip_load<BITS>(live ? wr : w0, woff, live ? (step * (SR / 32) + w * 4) * (BITS * 4) : 0, wv[slot]);
+    load_codes<BITS>(live ? wr : w0, woff, live ? (step * (SR / 32) + w * 4) * (BITS * 4) : 0, wv[slot]);
   };
 
   // activations: thread t stages chunk t % CPR of rows t / CPR + XROWS i
@@ -299,7 +263,7 @@ __global__ __launch_bounds__(512, 2) void qmm_strip_kernel(const StripArgs a) {
               for (int j = 0; j < 4; j++)
 #pragma unroll
                 for (int h = 0; h < 4; h++) {
-                  const uint32_t q0 = strip_code<BITS>(wv[slot], 8 * j + 2 * h), q1 = strip_code<BITS>(wv[slot], 8 * j + 2 * h + 1);
+                  const uint32_t q0 = code_at<BITS>(wv[slot], 8 * j + 2 * h), q1 = code_at<BITS>(wv[slot], 8 * j + 2 * h + 1);
                   if constexpr (BIG) {
                     o[j][h] = strip_pack<XT>(__builtin_fmaf(sc, (float)q0, bi), __builtin_fmaf(sc, (float)q1, bi));
                   } else {

@@ -99,12 +99,14 @@ __global__ __launch_bounds__(64 * NWM * NWN) void qmm_tile_kernel(const QmmArgs 
   constexpr int TM = BM / NWM, TN = BN / NWN;  // wave tile
   constexpr int FM = TM / 32, FN = TN / 32;  // 32 x 32 MFMA tiles per wave
   constexpr bool AFF = FMT != MXFP4;
-  constexpr int BITS = FMT == AFF8 ? 8 : 4;
+  constexpr bool ODD = FMT >= kAffOdd;       // affine codes of 2, 3, 5 or 6 bits
+  constexpr int BITS = fmt_bits(FMT);
   constexpr int RS = BK;                     // LDS row stride (bf16): 128 bytes, swizzled
   constexpr int XL = BM * BK * 2 / 16 / NT;  // 16-byte activation loads per thread and K-step
   // weight piece per thread and load: 16 bytes, or 8 when a K-step of the
   // tile's weights is less than 16 bytes per thread (256 x 128, 8 waves, 4-bit)
-  constexpr int PB = BN * BK * BITS / 8 / NT >= 16 ? 16 : 8;
+  // (ODD: 32 codes, BITS words)
+  constexpr int PB = ODD ? BITS * 4 : BN * BK * BITS / 8 / NT >= 16 ? 16 : 8;
   constexpr int PW = PB / 4;                 // words per piece
   constexpr int WT = BK * BITS / 8 / PB;     // threads per weight row and K-step
   constexpr int WROWS = NT / WT;             // weight rows per pass
@@ -112,7 +114,8 @@ __global__ __launch_bounds__(64 * NWM * NWN) void qmm_tile_kernel(const QmmArgs 
   constexpr int VPL = PB * 8 / BITS;         // values per weight load
   constexpr int CHG = AFF ? 8 : 16;          // groups in a 16-byte scale chunk
   static_assert(WP >= 1 && WROWS * WP == BN && BN <= NT && XL >= 1, "tile shape");
-  static_assert(PB == 16 || (BITS == 4 && PB == 8), "8-byte pieces only for 4-bit codes");
+  static_assert(ODD || PB == 16 || (BITS == 4 && PB == 8), "8-byte pieces only for 4-bit codes");
+  static_assert(!ODD || WP == 1, "one 32-code piece per thread");
 
   // double-buffered activation and dequantized-weight tiles; after the last
   // K-step the same bytes stage the output tile
@@ -269,11 +272,13 @@ __global__ __launch_bounds__(64 * NWM * NWN) void qmm_tile_kernel(const QmmArgs 
     }
   };
 
-  u32x4 xreg[XL], wreg[WP];
+  u32x4 xreg[XL], wreg[ODD ? 1 : WP];
+  uint32_t wodd[ODD ? BITS : 1];
   auto load_step = [&](int ks) {
     const int k0 = ks * BK;
+    if constexpr (ODD) load_codes<BITS>(wr, woff[0] + (uint32_t)(k0 / 8 * BITS), 0, wodd);
 #pragma unroll
-    for (int p = 0; p < WP; p++) {
+    for (int p = 0; p < (ODD ? 0 : WP); p++) {
       if constexpr (PB == 16) {
         wreg[p] = __builtin_bit_cast(
             u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, woff[p] + (uint32_t)(k0 * BITS / 8), 0, 0));
@@ -315,8 +320,18 @@ __global__ __launch_bounds__(64 * NWM * NWN) void qmm_tile_kernel(const QmmArgs 
 #pragma unroll
     for (int i = 0; i < XL; i++)
       if (i * NPART / XL == p) *reinterpret_cast<u32x4*>(&xs[buf][xdst(i)]) = xreg[i];
+    if constexpr (ODD) {  // codes 8 p .. 8 p + 7 of the piece
+      const uint32_t sb = sbw[0];
+      const float sc = xt_to_f32<XT>(sb & 0xFFFFu), bi = xt_to_f32<XT>(sb >> 16);
+      u32x4 o;
 #pragma unroll
-    for (int e = 0; e < NWORD; e++) {
+      for (int h = 0; h < 4; h++)
+        o[h] = pack_xt2<XT>(__builtin_fmaf(sc, (float)code_at<BITS>(wodd, 8 * p + 2 * h), bi),
+                            __builtin_fmaf(sc, (float)code_at<BITS>(wodd, 8 * p + 2 * h + 1), bi));
+      *reinterpret_cast<u32x4*>(&wsm[buf][wrow * RS] + (((4 * wpc + p) ^ swz(wrow)) << 3)) = o;
+    }
+#pragma unroll
+    for (int e = 0; e < (ODD ? 0 : NWORD); e++) {
       if (e * NPART / NWORD != p) continue;
       const int pp = e / PW;  // which weight load
       const int r = wrow + WROWS * pp;
@@ -704,5 +719,13 @@ __global__ __launch_bounds__(64 * NWM * NWN) void qmm_tile_kernel(const QmmArgs 
   if (a.ksplit > 1) store_partials(z);
   else store_out();
 }
+
+// 2-, 3-, 5- and 6-bit codes (qmm_odd.hip): tiles 4 (256 x 256, 8 waves) and
+// 6 (128 x 128, 4 waves), where every thread dequantizes one 32-code piece
+// (its BITS words, one group) per K-step, at 3.5 VALU instructions per code
+// against 2.9 for 4-bit codes.  MI355X, 14336 x 4096 6-bit g64: 512 rows 89
+// us, 2048 rows 251 (0.38 of 2.5 PF), against 493 us and 1.4 ms on the
+// general tile kernel, whose rounding of the weights this one shares.
+void qmm_launch_odd(int bits, const QmmArgs& a, int tile, int ksplit, hipStream_t stream);
 
 }  // namespace mlxq
