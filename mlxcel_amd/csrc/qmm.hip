@@ -304,7 +304,7 @@ QmmPlan qmm_plan(int fmt, int gs, int64_t M, int64_t N, int64_t K, int num_cus, 
   int tile, ks_planned = 0;
   if (tile_req >= 0 && tile_req < kTiles) {
     tile = tile_req;
-  } else if (fit_round && odd) {
+  } else if (fit_round && (odd || (M > 128 && M <= 1024 && tiles_of(4) <= num_cus))) {
     tile = plan_mid(odd, M, N, nks, num_cus, ks_planned);
   } else {
     // 256 x 256 (8 waves) when there are enough tiles or K is long enough

@@ -32,3 +32,15 @@ def test_edges(monkeypatch, bits, dt, M, N, K, gs, tile, ks):
     (wq, s, b), (wqn, sv, bv) = _weights(rng, (N,), K, bits, gs, dt)
     y = mq.quantized_matmul(x, wq, s, b, True, gs, bits)
     assert _rel(y, og.qmm(xv, wqn, sv, bv, True, gs, bits), dt) <= 1e-2
+
+
+@pytest.mark.parametrize("bits,dt", [(4, "bfloat16"), (8, "bfloat16"), (4, "float16")])
+@pytest.mark.parametrize("M,N,K,gs", [(129, 1900, 1152, 64), (333, 770, 4096, 64), (768, 600, 2048, 128), (1024, 129, 576, 32)])
+def test_splits_that_fill_a_round(bits, dt, M, N, K, gs):
+    # 4- and 8-bit codes take the same tile and K-split choice at 129-1024 rows
+    rng = np.random.default_rng(47000 + bits + M)
+    announce("qmm mid plan", bits, dt, M, N, K, gs)
+    x, xv = _dev(rng.standard_normal((M, K)), dt)
+    (wq, s, b), (wqn, sv, bv) = _weights(rng, (N,), K, bits, gs, dt)
+    y = mq.quantized_matmul(x, wq, s, b, True, gs, bits)
+    assert _rel(y, og.qmm(xv, wqn, sv, bv, True, gs, bits), dt) <= 1e-2
