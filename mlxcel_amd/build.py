@@ -16,6 +16,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libmlxq.so")
+NATIVE = os.path.join(HERE, "_mlxq_native.so")
 # bench.py's streaming-read reference kernel, kept out of the C-ABI library
 BENCH_LIB = os.path.join(HERE, "libmlxq_bench.so")
 BENCH_SOURCES = {"bench_read.hip": []}
@@ -196,6 +197,28 @@ def _verify_b4_mfma_chains() -> None:
     check_b4_mfma_chains(open(B4_ASM).read())
 
 
+def _build_native() -> None:
+    """The Python entry points' native module (host code only, against torch's
+    C++ headers and libmlxq.so beside it)."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-w",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[f"-I{p}" for p in cpp_extension.include_paths()], "-I/opt/rocm/include",
+           "-I" + sysconfig.get_paths()["include"], os.path.join(CSRC, "pyext.cpp"), "-o", NATIVE + ".tmp",
+           f"-L{libs}", "-ltorch_python", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip",
+           f"-L{HERE}", "-l:libmlxq.so", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for pyext.cpp:\n{' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+    os.replace(NATIVE + ".tmp", NATIVE)
+
+
 def build(verbose: bool = True) -> str:
     """Compile every source and link libmlxq.so; always rebuilds."""
     if not os.path.exists(HIPCC) and shutil.which("hipcc") is None:
@@ -210,6 +233,7 @@ def build(verbose: bool = True) -> str:
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
     os.replace(tmp, LIB)
+    _build_native()
     _verify_group_ring_waits()
     _verify_b4_mfma_chains()
     bobjs = [_compile(k, v) for k, v in BENCH_SOURCES.items()]

@@ -11,15 +11,29 @@ reference's message; combinations this library does not implement raise
 
 Torch is used only for device memory and the current HIP stream; all
 arithmetic happens in the HIP kernels.
+
+Each wrapper hands its arguments to the native module first (csrc/pyext.cpp:
+exact torch tensors on a HIP device, plain Python numbers); where that returns
+None the call takes the ctypes binding below, which also reports the errors.
 """
 from __future__ import annotations
 
 import ctypes
+import os
 from typing import Optional, Sequence
 
 import torch
 
 from . import _lib
+
+if os.path.exists(_lib.NATIVE_PATH):
+    from . import _mlxq_native as _native
+else:  # not built: _lib.load() raises at the first call
+
+    class _native:
+        quantized_matmul = quantized_matmul_multi = gather_qmm = staticmethod(lambda *a: None)
+        dequantize = quantize = fused_moe = staticmethod(lambda *a: None)
+
 
 _TORCH_TO_MLXQ = {
     torch.bool: _lib.BOOL,
@@ -73,6 +87,13 @@ def _raise(status: int) -> None:
     raise QuantizedOpError(f"status {status}: {msg}")
 
 
+def _done(r):
+    """The native module's result, or the error of its status code."""
+    if type(r) is int:
+        _raise(r)
+    return r
+
+
 def _stream(device: torch.device) -> ctypes.c_void_p:
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
@@ -100,6 +121,9 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor,
                      group_size: Optional[int] = None, bits: Optional[int] = None,
                      mode: str = "affine", *, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``x @ dequantize(w, scales, biases).T`` (``transpose=True``), as ``mx.quantized_matmul``."""
+    r = _native.quantized_matmul(x, w, scales, biases, None, False, transpose, group_size, bits, mode, out)
+    if r is not None:
+        return _done(r)
     lib = _lib.load()
     ax, aw, as_, ab = _arr(x), _arr(w), _arr(scales), _arr(biases)
     gs, b = _opt(group_size), _opt(bits)
@@ -125,6 +149,9 @@ def quantized_linear(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
                      bits: Optional[int] = None, mode: str = "affine", *,
                      out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """The reference's ``quantized_linear_forward``: ``x @ W^T + linear_bias``."""
+    r = _native.quantized_matmul(x, w, scales, biases, linear_bias, True, True, group_size, bits, mode, out)
+    if r is not None:
+        return _done(r)
     lib = _lib.load()
     gs, b = _opt(group_size), _opt(bits)
     ax, aw, as_, ab, alb = _arr(x), _arr(w), _arr(scales), _arr(biases), _arr(linear_bias)
@@ -160,6 +187,9 @@ def quantized_matmul_multi(x: torch.Tensor, ws: Sequence[torch.Tensor], scales: 
                            out: Optional[Sequence[torch.Tensor]] = None) -> list:
     """``[quantized_matmul(x, w_i, s_i, b_i) for i]`` (transpose=True) in one
     call; at decode sizes one launch that reads x once (q/k/v, gate/up)."""
+    r = _native.quantized_matmul_multi(x, ws, scales, biases, group_size, bits, mode, out)
+    if r is not None:
+        return _done(r)
     lib = _lib.load()
     n = len(ws)
     gs, b = _opt(group_size), _opt(bits)
@@ -197,6 +227,10 @@ def gather_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor,
                group_size: Optional[int] = None, bits: Optional[int] = None, mode: str = "affine",
                sorted_indices: bool = False, *, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``out[i] = x[lhs[i]] @ dequantize(w[rhs[i]]).T``, as ``mx.gather_qmm``."""
+    r = _native.gather_qmm(x, w, scales, biases, lhs_indices, rhs_indices, transpose, group_size, bits, mode,
+                           sorted_indices, out)
+    if r is not None:
+        return _done(r)
     lib = _lib.load()
     ax, aw, as_, ab = _arr(x), _arr(w), _arr(scales), _arr(biases)
     al, ar = _arr(lhs_indices), _arr(rhs_indices)
@@ -240,6 +274,9 @@ def dequantize(w: torch.Tensor, scales: torch.Tensor, biases: Optional[torch.Ten
         shape[-1] = shape[-1] * 32 // b
         odt = dtype if dtype is not None else (scales.dtype if mode == "affine" else torch.bfloat16)
         out = torch.empty(shape, dtype=odt, device=_device_of(w))
+    r = _native.dequantize(w, scales, biases, gs, b, mode, dcode, out)
+    if r is not None:
+        return _done(r)
     aw, as_, ab, ao = _arr(w), _arr(scales), _arr(biases), _arr(out)
     dev = _device_of(w)
     with torch.cuda.device(dev):
@@ -271,6 +308,11 @@ def quantize(w: torch.Tensor, group_size: Optional[int] = None, bits: Optional[i
         else:
             scales = torch.empty(sshape, dtype=torch.uint8, device=dev)
             biases = None
+    r = _native.quantize(w, group_size, bits, mode, wq, scales, biases)
+    if r is not None:
+        if r is not True:
+            _raise(r)
+        return (wq, scales, biases) if mode == "affine" else (wq, scales)
     aw, aq, as_, ab = _arr(w), _arr(wq), _arr(scales), _arr(biases)
     with torch.cuda.device(dev):
         st = lib.mlxq_quantize(_ref(aw), _opt(group_size), _opt(bits), _mode(mode), _ref(aq), _ref(as_),
@@ -283,6 +325,10 @@ def quantize(w: torch.Tensor, group_size: Optional[int] = None, bits: Optional[i
 def _fused_moe(fn_name: str, x, indices, gate_w, gate_s, gate_b, up_w, up_s, up_b, down_w, down_s, down_b,
                scores, din: int, dff: int, k: int, gu_bits: int, d_bits: int, group_size: int,
                out: Optional[torch.Tensor]) -> torch.Tensor:
+    r = _native.fused_moe(fn_name == "mlxq_fused_moe_geglu", x, indices, gate_w, gate_s, gate_b, up_w, up_s, up_b,
+                          down_w, down_s, down_b, scores, din, dff, k, gu_bits, d_bits, group_size, out)
+    if r is not None:
+        return _done(r)
     lib = _lib.load()
     dev = _device_of(x)
     if out is None:

@@ -1,0 +1,95 @@
+"""The entry points' native module (csrc/pyext.cpp) against the ctypes path it
+stands in for: the same bytes for every wrapper, the same errors, and the
+argument forms it hands back (tensor subclasses, other Python number types,
+torch-function modes, CPU tensors)."""
+import numpy as np
+import pytest
+import torch
+
+import mlxcel_amd as mq
+from mlxcel_amd import ops
+from test_gpu_strip import _weights
+
+pytestmark = pytest.mark.gpu
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+def _both(monkeypatch, f):
+    native = f()
+    with monkeypatch.context() as m:
+        for name in ("quantized_matmul", "quantized_matmul_multi", "gather_qmm", "dequantize", "quantize", "fused_moe"):
+            m.setattr(ops._native, name, lambda *a: None)
+        return native, f()
+
+
+def _flat(r):
+    return list(r) if isinstance(r, (list, tuple)) else [r]
+
+
+def test_same_results_as_the_ctypes_path(monkeypatch):
+    rng = np.random.default_rng(48000)
+    E, N, K = 4, 64, 128
+    x = torch.from_numpy(rng.standard_normal((3, K)).astype(np.float32)).to(torch.bfloat16).cuda()
+    (w, s, b), _ = _weights(rng, (N,), K, 4, 64, "bfloat16")
+    (we, se, be), _ = _weights(rng, (E, N), K, 4, 64, "bfloat16")
+    (wg, sg, bg), _ = _weights(rng, (E, N), K, 4, 64, "bfloat16")
+    (wd, sd, bd), _ = _weights(rng, (E, K), N, 4, 64, "bfloat16")
+    lin = torch.ones(N, dtype=torch.bfloat16, device="cuda")
+    ids = torch.tensor([[2, 0], [1, 3], [0, 1]], device="cuda")
+    score = torch.tensor([0.25, 0.75], device="cuda")
+    side = torch.cuda.Stream()
+
+    def on_side():
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            y = mq.quantized_matmul(x, w, s, b)
+        torch.cuda.current_stream().wait_stream(side)
+        return y
+
+    for f in (lambda: mq.quantized_matmul(x, w, s, b), on_side,
+              lambda: mq.quantized_matmul(x[None], w, s, b, True, 64, 4, "affine"),
+              lambda: mq.quantized_matmul(x, w, s, b, group_size=np.int64(64), bits=4),
+              lambda: mq.quantized_matmul(x.as_subclass(_Sub), w, s, b).as_subclass(torch.Tensor),
+              lambda: mq.quantized_matmul(x, w, s, b, out=torch.empty(3, N, dtype=torch.bfloat16, device="cuda")),
+              lambda: mq.quantized_linear(x, w, s, b, lin), lambda: mq.quantized_linear(x, w, s, b),
+              lambda: mq.quantized_matmul_multi(x, [w, w], (s, s), [b, b]),
+              lambda: mq.gather_qmm(x.view(3, 1, 1, K), we, se, be, None, ids),
+              lambda: mq.dequantize(w, s, b), lambda: mq.quantize(lin.expand(4, N).contiguous()),
+              lambda: mq.fused_moe_expert(x[0], ids[0], wg, sg, bg, we, se, be, wd, sd, bd, score, K, N, 2, 4, 4, 64)):
+        got, want = _both(monkeypatch, f)
+        assert type(got) is type(want)
+        for g, h in zip(_flat(got), _flat(want)):
+            assert g.shape == h.shape and g.dtype == h.dtype and torch.equal(g.view(torch.uint8), h.view(torch.uint8))
+
+
+@pytest.mark.parametrize("change", ["w_dtype", "no_biases", "inner", "mode", "out_shape", "cpu", "bits"])
+def test_same_errors_as_the_ctypes_path(monkeypatch, change):
+    rng = np.random.default_rng(49000)
+    x = torch.ones((2, 128), dtype=torch.bfloat16, device="cuda")
+    (w, s, b), _ = _weights(rng, (8,), 128, 4, 64, "bfloat16")
+    a = dict(x=x, w=w, scales=s, biases=b)
+    if change == "w_dtype":
+        a["w"] = w.view(torch.int32)
+    elif change == "no_biases":
+        a["biases"] = None
+    elif change == "inner":
+        a["x"] = x[:, :64].contiguous()
+    elif change == "mode":
+        a["mode"] = "nonsense"
+    elif change == "out_shape":
+        a["out"] = torch.empty((3, 8), dtype=torch.bfloat16, device="cuda")
+    elif change == "cpu":
+        a["x"] = x.cpu()
+    else:
+        a["bits"] = 7
+
+    def message():
+        with pytest.raises((ValueError, NotImplementedError, ops.QuantizedOpError)) as e:
+            mq.quantized_matmul(**a)
+        return type(e.value), str(e.value)
+
+    got, want = _both(monkeypatch, message)
+    assert got == want and got[1]
