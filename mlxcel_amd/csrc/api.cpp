@@ -1366,7 +1366,8 @@ bool try_strip(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, cons
     // kernels forced by other switches stay forced
     if (!kn.qmv_kernel.empty() || kn.qmm_tile >= 0 || kn.qmm_ksplit > 0 || kn.gen_ks > 0 || kn.qmm_min_rows != kQmmMinRows)
       return false;
-    if (rows < (odd ? 5 : 17) || rows > 128) return false;
+    // (odd widths whose K the prefill tiles do not take: in passes of 128 rows)
+    if (rows < (odd ? 5 : 17) || rows > (odd && sp.K % 64 != 0 ? 1024 : 128)) return false;
     if (sp.out_dtype == MLXQ_BFLOAT16 && !odd && !rounds_weights(sp)) return false;
   }
   const int dev = current_device();
@@ -1374,6 +1375,10 @@ bool try_strip(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, cons
   const int fmt = sp.mode == MXFP4_M ? mlxq::MXFP4 : mlxq::AFF4;
   mlxq::StripPlan p = mlxq::strip_plan(fmt, sp.bits, sp.gs, rows, sp.N, sp.K, 0, cus, kn.strip_nwn, kn.strip_mt, kn.strip_ks);
   if (!p.ok || (!forced && !odd && rows > 64 && p.windows > 4)) return false;
+  // several passes only where they fill half the CUs (6-bit, 512 rows: 4096 x
+  // 4128 91 us vs 267 on the general kernel; 1000 rows over 1100 x 544, 54
+  // workgroups, 85 vs 28)
+  if (!forced && rows > 128 && (int64_t)p.row_blocks * p.ks * 2 < cus) return false;
   auto part = [&] { return (size_t)p.ks * rows * sp.N * sizeof(float); };
   // partials that cannot be had here: the kernels below
   if (p.ks > 1 && !scratch_fits(dev, stream, part(), ss)) return false;
@@ -1401,7 +1406,7 @@ bool try_strip(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, cons
 // workgroup per 64 weight rows of an expert finds the expert's entries in
 // the indices itself.  MI355X, 128 experts of 768 x 2048 4-bit, top 8,
 // against grouping on the device + 16x16-MFMA tiles: 128 tokens 41 us vs
-// 104, 512 tokens 79 vs 119, 1024 tokens 117 vs 180; 8 experts of 4096 x
+// 104, 512 tokens 57 vs 119, 1024 tokens 100 vs 180; 8 experts of 4096 x
 // 2048 8-bit, top 2: 64 tokens 20 vs 65, 1024 tokens 114 vs 211.
 bool try_strip_gather(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, const mlxq_array* scales,
                       const mlxq_array* biases, const DirectIdx& dl, const DirectIdx& dr, mlxq_array* out, int64_t B,

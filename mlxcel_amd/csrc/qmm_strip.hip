@@ -15,9 +15,10 @@ size_t strip_lds(int mt, int nwn, int gs) {
 
 // Microseconds of a launch on MI355X: start + per-window time of a wave
 // (fitted to graph-timed 4-bit g64 calls over 11 shapes from 1024 x 4096 to
-// 28672 x 4096; 3- and 6-bit codes lie within 15%), [log2(mt)][log2(nwn)].
-constexpr float kStart[4][3] = {{4.0f, 5.0f, 3.6f}, {4.7f, 4.1f, 3.2f}, {0.f, 4.9f, 3.9f}, {0.f, 0.f, 4.2f}};
-constexpr float kWindow[4][3] = {{1.0f, 0.65f, 0.70f}, {1.3f, 1.1f, 0.98f}, {0.f, 1.53f, 1.21f}, {0.f, 0.f, 2.4f}};
+// 28672 x 4096; 3- and 6-bit codes lie within 15%), [kTilesM index][log2(nwn)].
+constexpr int kTilesM[5] = {1, 2, 3, 4, 8};  // 16-row activation tiles per pass
+constexpr float kStart[5][3] = {{4.0f, 5.0f, 3.6f}, {4.7f, 4.1f, 3.2f}, {0.f, 4.5f, 3.5f}, {0.f, 4.9f, 3.9f}, {0.f, 0.f, 4.2f}};
+constexpr float kWindow[5][3] = {{1.0f, 0.65f, 0.70f}, {1.3f, 1.1f, 0.98f}, {0.f, 1.32f, 1.10f}, {0.f, 1.53f, 1.21f}, {0.f, 0.f, 2.4f}};
 
 }  // namespace
 
@@ -28,15 +29,17 @@ StripPlan strip_plan(int fmt, int bits, int gs, int64_t rows, int64_t N, int64_t
   if (rows * K * 2 >= ((int64_t)1 << 31) || N * (K / 32) * bits * 4 >= ((int64_t)1 << 31) || N * (K / gs) * 2 >= ((int64_t)1 << 31))
     return p;
   const int64_t per = experts > 0 ? (rows + experts - 1) / experts : rows;
-  int lm = per <= 16 ? 0 : per <= 32 ? 1 : per <= 64 ? 2 : 3;
+  int lm = per <= 16 ? 0 : per <= 32 ? 1 : per <= 48 ? 2 : per <= 64 ? 3 : 4;
   // an expert's rows spread around the average and are taken 16 mt at a
-  // time: 32 at a time measured fastest from 12 to ~100 rows per expert (128
-  // experts of 768 x 2048, 64 rows each: 117 us vs 135 with 64 at a time),
-  // 128 past that (8 experts of 4096 x 2048, 256 rows each: 114 vs 127)
-  if (experts > 0) lm = per <= 11 ? 0 : per <= 100 ? 1 : 3;
-  for (int i = 0; i < 4; i++)
-    if (mt_req == 1 << i) lm = i;
-  const int mt = 1 << lm;
+  // time: 48 at a time measured fastest from 25 to ~100 rows per expert (128
+  // experts of 768 x 2048, 32 rows each: 57 us, 79 with 32 at a time, 83 with
+  // 64; 64 rows each 100, 118, 137), 32 below that (16 rows each 48.6 us vs
+  // 52.3), 128 past it (8 experts of 4096 x 2048, 256 rows each: 114 vs 127
+  // with 32)
+  if (experts > 0) lm = per <= 11 ? 0 : per <= 24 ? 1 : per <= 100 ? 2 : 4;
+  for (int i = 0; i < 5; i++)
+    if (mt_req == kTilesM[i]) lm = i;
+  const int mt = kTilesM[lm];
   const int64_t passes = experts > 0 ? 1 : (rows + 16 * mt - 1) / (16 * mt);
   float best = 0.f;
   for (int ln = 0; ln < 3; ln++) {

@@ -28,7 +28,7 @@
 // first loads, sum over the K waves), the dequantization (2.6 VALU per code)
 // adds 2.5, staging and barriers 2; the 25.7 MB of weights (3.2 us at 8 TB/s)
 // hide under these.  Per 128-position window a wave spends 0.70 us at 16
-// activation rows, 0.98 at 32, 1.21 at 64 and 2.4 at 128.  Two windows per
+// activation rows, 0.98 at 32, 1.10 at 48, 1.21 at 64 and 2.4 at 128.  Two windows per
 // step (one past 16 rows) and a ring of two steps measured best of 1, 2 and
 // 4 windows and rings of 2 to 8; two workgroups per CU instead of one
 // changed nothing.
@@ -379,6 +379,8 @@ hipError_t strip_launch_fmt(const StripArgs& a, const StripPlan& p, dim3 grid, h
   STRIP_CASE(2, 1)
   STRIP_CASE(2, 2)
   STRIP_CASE(2, 4)
+  STRIP_CASE(3, 2)
+  STRIP_CASE(3, 4)
   STRIP_CASE(4, 2)
   STRIP_CASE(4, 4)
   STRIP_CASE(8, 4)

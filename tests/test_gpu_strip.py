@@ -45,7 +45,7 @@ def _rel(y, want, dt):
 @pytest.mark.parametrize("dt", ["bfloat16", "float16"])
 @pytest.mark.parametrize("M,N,K,gs,nwn,ks", [
     (5, 33, 32, 32, 4, 1), (16, 64, 160, 32, 2, 1), (16, 17, 1056, 32, 1, 2), (17, 65, 4096, 128, 4, 3),
-    (32, 1, 192, 64, 1, 1), (33, 130, 2112, 64, 2, 2), (64, 100, 640, 128, 4, 1), (65, 48, 1088, 64, 4, 2),
+    (32, 1, 192, 64, 1, 1), (33, 130, 2112, 64, 2, 2), (64, 100, 640, 128, 4, 1), (65, 48, 1088, 64, 4, 2), (48, 80, 1088, 64, 2, 2), (35, 65, 416, 32, 4, 1),
     (128, 70, 576, 64, 4, 1), (300, 40, 256, 32, 4, 1)])
 def test_dense_edges(monkeypatch, bits, dt, M, N, K, gs, nwn, ks):
     setknob(monkeypatch, "MLXQ_STRIP", "2")
@@ -59,7 +59,7 @@ def test_dense_edges(monkeypatch, bits, dt, M, N, K, gs, nwn, ks):
     assert _rel(y, og.qmm(xv, wqn, sv, bv, True, gs, bits), dt) <= 1e-2
 
 
-@pytest.mark.parametrize("bits,M", [(3, 5), (6, 128), (4, 17), (8, 64), (4, 100)])
+@pytest.mark.parametrize("bits,M", [(3, 5), (6, 128), (4, 17), (8, 64), (4, 100), (5, 40)])
 def test_default_route_matches_other_kernels(monkeypatch, bits, M):
     rng = np.random.default_rng(42000 + bits)
     N, K, gs = 513, 4096, 64
@@ -120,7 +120,7 @@ def test_mxfp4_special_scales(monkeypatch):
 
 
 @pytest.mark.parametrize("bits,gs", [(4, 64), (8, 32), (4, 128)])
-@pytest.mark.parametrize("counts", [[8, 8, 8, 8], [0, 40, 1, 0, 33, 16], [0, 0, 130, 0, 300], [64, 0]])
+@pytest.mark.parametrize("counts", [[8, 8, 8, 8], [0, 40, 1, 0, 33, 16], [0, 0, 130, 0, 300], [64, 0], [30, 49, 20, 96]])
 @pytest.mark.parametrize("idx", [torch.int32, torch.int64])
 def test_sorted_gather(bits, gs, counts, idx):
     rng = np.random.default_rng(45000 + bits + sum(counts))
@@ -132,3 +132,15 @@ def test_sorted_gather(bits, gs, counts, idx):
     y = mq.gather_qmm(x, wq, s, b, None, torch.from_numpy(ids).to(idx).cuda(), True, gs, bits, "affine", True)
     want = np.stack([og.qmm(xv[i], wqn[e], sv[e], bv[e], True, gs, bits) for i, e in enumerate(ids)])
     assert _rel(y, want, "bfloat16") <= 1e-2
+
+
+@pytest.mark.parametrize("bits,dt", [(6, "bfloat16"), (3, "float16")])
+def test_rows_in_passes(bits, dt):
+    # more than 128 rows of an odd width whose K the prefill tiles do not take
+    rng = np.random.default_rng(46500 + bits)
+    M, N, K, gs = 200, 2080, 4128, 32
+    announce("strip passes", bits, dt)
+    x, xv = _dev(rng.standard_normal((M, K)), dt)
+    (wq, s, b), (wqn, sv, bv) = _weights(rng, (N,), K, bits, gs, dt)
+    y = mq.quantized_matmul(x, wq, s, b, True, gs, bits)
+    assert _rel(y, og.qmm(xv, wqn, sv, bv, True, gs, bits), dt) <= 1e-2
