@@ -147,8 +147,10 @@ const char* mlxq_version(void);
  * with transpose=true run the specialised kernels, and so does float16
  * (x, scales, biases and result) 4/8-bit affine with transpose=true (decode
  * and prefill; its prefill dequantizes the weights to float16, as the
- * reference's dequantize + GEMM route does); every other combination runs
- * the general path: affine calls of 1-4 rows per matrix with transpose=true
+ * reference's dequantize + GEMM route does).  Affine codes of 2, 3, 5 and 6
+ * bits with bfloat16 or float16 x, scales and biases of one type and
+ * transpose=true run the specialised kernels from 5 rows on.  Every other
+ * combination runs the general path: affine calls of 1-4 rows per matrix with transpose=true
  * (1-2 with transpose=false) on its row-streaming decode kernels (fp32
  * products, no weight rounding), the rest on its tile kernel (float16
  * results there also round the dequantized weights to float16).  Operands
