@@ -11,7 +11,8 @@ import os
 
 MAX_DIMS = 8
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libmlxq.so")
-NATIVE_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_mlxq_native.so")  # csrc/pyext.cpp
+# the entry points' native module (csrc/pyext.cpp); without it they use this binding
+NATIVE_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_mlxq_native.so")
 
 # mlxq_status
 OK, EINVAL, EUNSUPPORTED, EHIP, ENOMEM = 0, 1, 2, 3, 4
@@ -67,8 +68,6 @@ def load() -> ctypes.CDLL:
         raise LibraryNotBuilt(
             f"{LIB_PATH} is missing: build it with `python -m mlxcel_amd.build` "
             "(the quantized matmul has no CPU fallback)")
-    if not os.path.exists(NATIVE_PATH):
-        raise LibraryNotBuilt(f"{NATIVE_PATH} is missing: build it with `python -m mlxcel_amd.build`")
     lib = ctypes.CDLL(LIB_PATH)
     A = ctypes.POINTER(MlxqArray)
     P = ctypes.c_void_p

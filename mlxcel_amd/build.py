@@ -208,7 +208,7 @@ def _build_native() -> None:
 
     libs = os.path.join(os.path.dirname(torch.__file__), "lib")
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-w",
-           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f'-DMLXQ_TORCH_VERSION="{torch.__version__}"',
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            *[f"-I{p}" for p in cpp_extension.include_paths()], "-I/opt/rocm/include",
            "-I" + sysconfig.get_paths()["include"], os.path.join(CSRC, "pyext.cpp"), "-o", NATIVE + ".tmp",

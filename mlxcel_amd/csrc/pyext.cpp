@@ -338,4 +338,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_mlxq_native", nullptr, -1, method
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__mlxq_native() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__mlxq_native() {
+  PyObject* m = PyModule_Create(&module);
+  // the torch it was compiled against: ops.py takes no other
+  if (m && PyModule_AddStringConstant(m, "torch_version", MLXQ_TORCH_VERSION) < 0) Py_CLEAR(m);
+  return m;
+}

@@ -14,26 +14,45 @@ arithmetic happens in the HIP kernels.
 
 Each wrapper hands its arguments to the native module first (csrc/pyext.cpp:
 exact torch tensors on a HIP device, plain Python numbers); where that returns
-None the call takes the ctypes binding below, which also reports the errors.
+None, or the module is missing or was built for another torch, the call takes
+the ctypes binding below, which also reports the errors.
 """
 from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 from typing import Optional, Sequence
 
 import torch
 
 from . import _lib
 
-if os.path.exists(_lib.NATIVE_PATH):
-    from . import _mlxq_native as _native
-else:  # not built: _lib.load() raises at the first call
 
-    class _native:
-        quantized_matmul = quantized_matmul_multi = gather_qmm = staticmethod(lambda *a: None)
-        dequantize = quantize = fused_moe = staticmethod(lambda *a: None)
+class _ctypes_only:
+    """Stands in for the native module: every call takes the ctypes binding."""
+    quantized_matmul = quantized_matmul_multi = gather_qmm = staticmethod(lambda *a: None)
+    dequantize = quantize = fused_moe = staticmethod(lambda *a: None)
 
+
+def _load_native():
+    """The native module where it is there and was built for this torch."""
+    if not os.path.exists(_lib.NATIVE_PATH):
+        return _ctypes_only
+    try:
+        from . import _mlxq_native as native
+
+        built_for = getattr(native, "torch_version", "(unknown)")
+        if built_for == torch.__version__:
+            return native
+        why = f"it was built for torch {built_for}, this is {torch.__version__}"
+    except ImportError as e:  # another torch or Python, or no libmlxq.so beside it
+        why = str(e)
+    warnings.warn(f"{_lib.NATIVE_PATH} is not used, calls go through ctypes: {why}")
+    return _ctypes_only
+
+
+_native = _load_native()
 
 _TORCH_TO_MLXQ = {
     torch.bool: _lib.BOOL,
