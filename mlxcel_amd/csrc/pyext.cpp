@@ -185,13 +185,23 @@ PyObject* quantized_matmul(PyObject*, PyObject* const* v, Py_ssize_t n) {
 
 constexpr int kMulti = 4;
 
+// A reference of the call's own: another thread may change the caller's list
+// while the GIL is released.
+struct Held {
+  PyObject* o = nullptr;
+  ~Held() { Py_XDECREF(o); }
+};
+
 // items of a list or tuple of at most kMulti tensors
-int items(PyObject* o, PyObject** to) {
+int items(PyObject* o, Held* to) {
   const bool l = PyList_CheckExact(o), t = PyTuple_CheckExact(o);
   if (!l && !t) throw NotHandled{};
   const Py_ssize_t n = l ? PyList_GET_SIZE(o) : PyTuple_GET_SIZE(o);
   if (n < 1 || n > kMulti) throw NotHandled{};
-  for (Py_ssize_t i = 0; i < n; i++) to[i] = l ? PyList_GET_ITEM(o, i) : PyTuple_GET_ITEM(o, i);
+  for (Py_ssize_t i = 0; i < n; i++) {
+    to[i].o = l ? PyList_GET_ITEM(o, i) : PyTuple_GET_ITEM(o, i);
+    Py_INCREF(to[i].o);
+  }
   return (int)n;
 }
 
@@ -200,7 +210,7 @@ PyObject* quantized_matmul_multi(PyObject*, PyObject* const* v, Py_ssize_t n) {
   return entry(n, 8, [&]() -> PyObject* {
     const at::Tensor& xt = tensor(v[0]);
     const Arr x = arr(v[0]);
-    PyObject *wo[kMulti], *so[kMulti], *bo[kMulti], *oo[kMulti];
+    Held wo[kMulti], so[kMulti], bo[kMulti], oo[kMulti];
     const int cnt = items(v[1], wo);
     if (items(v[2], so) != cnt) throw NotHandled{};
     const bool biases = v[3] != Py_None, given = v[7] != Py_None;
@@ -212,15 +222,15 @@ PyObject* quantized_matmul_multi(PyObject*, PyObject* const* v, Py_ssize_t n) {
     mlxq_array* po[kMulti];
     at::Tensor out[kMulti];
     for (int i = 0; i < cnt; i++) {
-      w[i] = arr(wo[i]);
-      s[i] = arr(so[i]);
+      w[i] = arr(wo[i].o);
+      s[i] = arr(so[i].o);
       if (!w[i].on || !s[i].on) throw NotHandled{};
-      if (biases) b[i] = arr(bo[i]);
+      if (biases) b[i] = arr(bo[i].o);
       pw[i] = w[i].p();
       ps[i] = s[i].p();
       pb[i] = b[i].p();
       if (given) {
-        o[i] = arr(oo[i]);
+        o[i] = arr(oo[i].o);
         if (!o[i].on) throw NotHandled{};
       } else {
         int32_t nd, dt;
@@ -237,7 +247,7 @@ PyObject* quantized_matmul_multi(PyObject*, PyObject* const* v, Py_ssize_t n) {
     });
     PyObject* r = PyList_New(cnt);
     if (!r) return nullptr;
-    for (int i = 0; i < cnt; i++) PyList_SET_ITEM(r, i, keep(given ? oo[i] : Py_None, out[i]));
+    for (int i = 0; i < cnt; i++) PyList_SET_ITEM(r, i, keep(given ? oo[i].o : Py_None, out[i]));
     return r;
   });
 }

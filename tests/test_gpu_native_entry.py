@@ -2,6 +2,9 @@
 stands in for: the same bytes for every wrapper, the same errors, and the
 argument forms it hands back (tensor subclasses, other Python number types,
 torch-function modes, CPU tensors)."""
+import sys
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -93,3 +96,35 @@ def test_same_errors_as_the_ctypes_path(monkeypatch, change):
 
     got, want = _both(monkeypatch, message)
     assert got == want and got[1]
+
+
+def test_multi_holds_the_outputs_of_a_list_that_changes():
+    # another thread empties the list while the call runs without the GIL
+    rng = np.random.default_rng(49500)
+    x = torch.ones((2, 128), dtype=torch.bfloat16, device="cuda")
+    (w, s, b), _ = _weights(rng, (8,), 128, 4, 64, "bfloat16")
+    want = mq.quantized_matmul(x, w, s, b)
+    lists, stop = [[]], threading.Event()
+
+    def empty():
+        while not stop.is_set():
+            lists[0].clear()
+
+    t = threading.Thread(target=empty)
+    t.start()
+    try:
+        for i in range(300):
+            outs = [torch.empty(2, 8, dtype=torch.bfloat16, device="cuda") for _ in range(3)]
+            lists[0] = outs
+            r = ops._native.quantized_matmul_multi(x, [w] * 3, [s] * 3, [b] * 3, None, None, "affine", outs)
+            # None: emptied before the call looked at it
+            assert r is None or all(torch.equal(y, want) for y in r)
+    finally:
+        stop.set()
+        t.join()
+    outs = [torch.empty(2, 8, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    held = [sys.getrefcount(o) for o in (w, s, b, *outs)]
+    r = ops._native.quantized_matmul_multi(x, [w] * 2, (s,) * 2, [b] * 2, None, None, "affine", outs)
+    assert all(y is o for y, o in zip(r, outs))
+    del r
+    assert [sys.getrefcount(o) for o in (w, s, b, *outs)] == held
