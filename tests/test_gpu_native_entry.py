@@ -1,7 +1,8 @@
 """The entry points' native module (csrc/pyext.cpp) against the ctypes path it
-stands in for: the same bytes for every wrapper, the same errors, and the
-argument forms it hands back (tensor subclasses, other Python number types,
-torch-function modes, CPU tensors)."""
+stands in for: the same bytes for every wrapper, the same errors, the caller's
+stream, and the argument forms it hands back (tensor subclasses, other Python
+number types, torch-function modes, CPU tensors).  Whether the module took a
+call is asserted each time."""
 import sys
 import threading
 
@@ -20,12 +21,25 @@ class _Sub(torch.Tensor):
     pass
 
 
-def _both(monkeypatch, f):
-    native = f()
+NAMES = ("quantized_matmul", "quantized_matmul_multi", "gather_qmm", "dequantize", "quantize", "fused_moe")
+
+
+def _both(monkeypatch, f, handled=True):
+    """f() through the native module and through ctypes; the native module
+    must have taken the call (handled) or handed it back as None."""
+    assert ops._native is not ops._ctypes_only
+    native, results = ops._native, []
     with monkeypatch.context() as m:
-        for name in ("quantized_matmul", "quantized_matmul_multi", "gather_qmm", "dequantize", "quantize", "fused_moe"):
-            m.setattr(ops._native, name, lambda *a: None)
-        return native, f()
+        for name in NAMES:
+            def record(*a, fn=getattr(native, name)):
+                results.append(fn(*a))
+                return results[-1]
+            m.setattr(native, name, record)
+        got = f()
+        assert len(results) == 1 and (results[0] is not None) == handled
+        for name in NAMES:
+            m.setattr(native, name, lambda *a: None)
+        return got, f()
 
 
 def _flat(r):
@@ -46,16 +60,29 @@ def test_same_results_as_the_ctypes_path(monkeypatch):
     side = torch.cuda.Stream()
 
     def on_side():
-        side.wait_stream(torch.cuda.current_stream())
+        # x is written on the side stream behind a wait of some 10 ms: a launch
+        # on any other stream would read zeros
+        late = torch.zeros_like(x)
+        torch.cuda.synchronize()
         with torch.cuda.stream(side):
-            y = mq.quantized_matmul(x, w, s, b)
-        torch.cuda.current_stream().wait_stream(side)
+            torch.cuda._sleep(1 << 24)
+            late.copy_(x)
+            y = mq.quantized_matmul(late, w, s, b)
+        side.synchronize()
+        assert torch.equal(y, mq.quantized_matmul(x, w, s, b))
         return y
 
-    for f in (lambda: mq.quantized_matmul(x, w, s, b), on_side,
-              lambda: mq.quantized_matmul(x[None], w, s, b, True, 64, 4, "affine"),
-              lambda: mq.quantized_matmul(x, w, s, b, group_size=np.int64(64), bits=4),
+    def in_mode():
+        with torch.device("cuda"):  # a torch-function mode
+            return mq.quantized_matmul(x, w, s, b)
+
+    # forms that the native module hands back
+    for f in (lambda: mq.quantized_matmul(x, w, s, b, group_size=np.int64(64), bits=4), in_mode,
               lambda: mq.quantized_matmul(x.as_subclass(_Sub), w, s, b).as_subclass(torch.Tensor),
+              lambda: mq.quantized_matmul(x, w, s, b, bits=np.int64(4))):
+        got, want = _both(monkeypatch, f, handled=False)
+        assert torch.equal(got, want)
+    for f in (lambda: mq.quantized_matmul(x, w, s, b), lambda: mq.quantized_matmul(x[None], w, s, b, True, 64, 4, "affine"),
               lambda: mq.quantized_matmul(x, w, s, b, out=torch.empty(3, N, dtype=torch.bfloat16, device="cuda")),
               lambda: mq.quantized_linear(x, w, s, b, lin), lambda: mq.quantized_linear(x, w, s, b),
               lambda: mq.quantized_matmul_multi(x, [w, w], (s, s), [b, b]),
@@ -66,6 +93,7 @@ def test_same_results_as_the_ctypes_path(monkeypatch):
         assert type(got) is type(want)
         for g, h in zip(_flat(got), _flat(want)):
             assert g.shape == h.shape and g.dtype == h.dtype and torch.equal(g.view(torch.uint8), h.view(torch.uint8))
+    on_side()
 
 
 @pytest.mark.parametrize("change", ["w_dtype", "no_biases", "inner", "mode", "out_shape", "cpu", "bits"])
@@ -94,7 +122,8 @@ def test_same_errors_as_the_ctypes_path(monkeypatch, change):
             mq.quantized_matmul(**a)
         return type(e.value), str(e.value)
 
-    got, want = _both(monkeypatch, message)
+    # (a tensor off the GPU is handed back: the ctypes path has the message)
+    got, want = _both(monkeypatch, message, handled=change != "cpu")
     assert got == want and got[1]
 
 
