@@ -140,9 +140,10 @@ PyObject* entry(Py_ssize_t n, Py_ssize_t want, F&& f) {
     Py_RETURN_NONE;
   } catch (const Status& s) {
     return PyLong_FromLong(s.code);
-  } catch (const c10::OutOfMemoryError&) {
-    Py_RETURN_NONE;  // the ctypes path raises torch's own exception
   } catch (const std::exception&) {
+    // torch's own (out of memory, or Python code that an allocation runs under
+    // a dispatch mode): the ctypes path meets it again and raises it
+    PyErr_Clear();
     Py_RETURN_NONE;
   }
 }

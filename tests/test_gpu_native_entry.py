@@ -12,6 +12,7 @@ import torch
 
 import mlxcel_amd as mq
 from mlxcel_amd import ops
+from torch.utils._python_dispatch import TorchDispatchMode
 from test_gpu_strip import _weights
 
 pytestmark = pytest.mark.gpu
@@ -157,3 +158,26 @@ def test_multi_holds_the_outputs_of_a_list_that_changes():
     assert all(y is o for y, o in zip(r, outs))
     del r
     assert [sys.getrefcount(o) for o in (w, s, b, *outs)] == held
+
+
+def test_an_exception_of_a_dispatch_mode_reaches_the_caller():
+    rng = np.random.default_rng(49600)
+    x = torch.ones((2, 128), dtype=torch.bfloat16, device="cuda")
+    (w, s, b), _ = _weights(rng, (8,), 128, 4, 64, "bfloat16")
+    seen = []
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            if self.refuse:
+                raise LookupError("no allocation here")
+            return func(*args, **(kwargs or {}))
+
+    with Mode() as mode:
+        mode.refuse = False
+        y = mq.quantized_matmul(x, w, s, b)
+        assert seen  # the result was allocated through the mode
+        mode.refuse = True
+        with pytest.raises(LookupError, match="no allocation"):
+            mq.quantized_matmul(x, w, s, b)
+    assert torch.equal(y, mq.quantized_matmul(x, w, s, b))
