@@ -319,14 +319,17 @@ __global__ __launch_bounds__(256) void affine_quant_kernel(const void* __restric
     if (sh + BITS > 32) words[wd + 1 < BITS ? wd + 1 : wd] |= c >> (32 - sh);
   }
   if (live) {
+    // the caller's array of words: aligned as words, no more
+    typedef uint32_t words4 __attribute__((ext_vector_type(4), aligned(4)));
+    typedef uint32_t words2 __attribute__((ext_vector_type(2), aligned(4)));
     uint32_t* d = wq + piece * BITS;
     if constexpr (BITS % 4 == 0) {
 #pragma unroll
       for (int i = 0; i < BITS / 4; i++)
-        reinterpret_cast<u32x4*>(d)[i] = u32x4{words[4 * i], words[4 * i + 1], words[4 * i + 2], words[4 * i + 3]};
+        reinterpret_cast<words4*>(d)[i] = words4{words[4 * i], words[4 * i + 1], words[4 * i + 2], words[4 * i + 3]};
     } else if constexpr (BITS % 2 == 0) {
 #pragma unroll
-      for (int i = 0; i < BITS / 2; i++) reinterpret_cast<u32x2*>(d)[i] = u32x2{words[2 * i], words[2 * i + 1]};
+      for (int i = 0; i < BITS / 2; i++) reinterpret_cast<words2*>(d)[i] = words2{words[2 * i], words[2 * i + 1]};
     } else {
 #pragma unroll
       for (int i = 0; i < BITS; i++) d[i] = words[i];
@@ -426,8 +429,9 @@ __global__ __launch_bounds__(256) void mxfp4_quant_kernel(const uint16_t* __rest
   // so is its distance to the two nearest code points, and the first minimum
   // is the smaller code: the code's magnitude is the number of midpoints the
   // value lies above (a midpoint itself goes down), a zero has code 0 whatever
-  // its sign.  Elsewhere (and for NaN and infinities, which reach the
-  // exponent) every code point is tried.
+  // its sign.  A NaN, which the maximum passes over, lies above none and has
+  // code 0, as where no distance compares smaller.  Elsewhere (and with an
+  // infinity, which reaches the exponent) every code point is tried.
   if (__ballot(e < -120 || e > 120) == 0ull) {
     const float mid[7] = {0.25f * p, 0.75f * p, 1.25f * p, 1.75f * p, 2.5f * p, 3.5f * p, 5.0f * p};
 #pragma unroll

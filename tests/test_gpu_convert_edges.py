@@ -3,12 +3,16 @@ quotients on and next to a rounding tie, scales whose reciprocal is not a
 normal number, values on the fp4 midpoints, shared exponents past the fast
 range, row counts around a workgroup's share of words (against the oracle's
 restatement of the reference's quantizers and dequantizers)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import mlxcel_amd as mq
 import oracle as orc
+from mlxcel_amd import _lib
+from mlxcel_amd.ops import _arr, _ref
 from helpers import announce, dev_bf16, dev_u8, dev_u32, host_u16
 
 pytestmark = pytest.mark.gpu
@@ -54,6 +58,24 @@ def test_mxfp4_quantize_midpoints_and_exponents():
     np.testing.assert_array_equal(sc.cpu().numpy(), esc)
 
 
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** 122, 2.0 ** -124])
+def test_mxfp4_quantize_nan_and_infinity_among_finite_values(scale):
+    announce("quantize mxfp4 nonfinite", scale)
+    rng = np.random.default_rng(51500)
+    w = rng.standard_normal((6, 96)).astype(np.float32) * np.float32(scale)
+    w[0, ::7], w[1, 5], w[2] = np.nan, -np.nan, np.nan
+    w[3, 40], w[4, 70] = np.inf, -np.inf
+    w[4, 71] = np.nan
+    bits = orc.f32_to_bf16(w)
+    ewq, esc = orc.mxfp4_quantize(bits)
+    wq, sc = mq.quantize(dev_bf16(bits), 32, 4, "mxfp4")
+    finite = ~np.isinf(w).reshape(6, 3, 32).any(-1)
+    # (a group with an infinity has no scale the reference defines)
+    np.testing.assert_array_equal(wq.cpu().view(torch.int32).numpy().view(np.uint32).reshape(6, 3, 4)[finite],
+                                  ewq.reshape(6, 3, 4)[finite])
+    np.testing.assert_array_equal(sc.cpu().numpy()[finite], esc.reshape(6, 3)[finite])
+
+
 @pytest.mark.parametrize("bits", [2, 4, 8])
 @pytest.mark.parametrize("rows,K", [(1, 128), (7, 256), (33, 1152), (65, 128)])
 def test_affine_dequantize_words_and_nonfinite(bits, rows, K):
@@ -75,3 +97,24 @@ def test_mxfp4_dequantize_uniform_scales(scale):
     sc = np.full((40, 8), scale, np.uint8)
     got = host_u16(mq.dequantize(dev_u32(wq), dev_u8(sc), None, 32, 4, "mxfp4"))
     np.testing.assert_array_equal(got, orc.mxfp4_dequantize(wq, sc))
+
+
+@pytest.mark.parametrize("bits", [1, 2, 3, 4, 5, 6, 8])
+def test_affine_quantize_into_words_aligned_as_words(bits):
+    # a caller of the C ABI may give any uint32 array for the codes
+    announce("quantize offset words", bits)
+    lib = _lib.load()
+    w = (torch.randn(9, 192, generator=torch.Generator().manual_seed(bits)) * 0.02).to(torch.bfloat16).cuda()
+    want, s, b = mq.quantize(w, 64, bits)
+    n = want.numel()
+    buf = torch.zeros(n + 8, dtype=torch.int32, device="cuda")
+    for off in (1, 2, 3):
+        wq = buf[off:off + n].view(want.shape).view(torch.uint32)
+        assert wq.data_ptr() % 16 == 4 * off
+        buf.zero_()
+        args = [_arr(t) for t in (w, wq, s, b)]
+        st = lib.mlxq_quantize(_ref(args[0]), 64, bits, b"affine", *[_ref(a) for a in args[1:]],
+                               ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert st == _lib.OK, _lib.last_error()
+        assert torch.equal(wq.view(torch.int32), want.view(torch.int32))
+        assert not buf[:off].any() and not buf[off + n:].any()
