@@ -1439,6 +1439,17 @@ bool try_strip_gather(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* 
   a.rhs = dr.p;
   a.rhs_stride = dr.stride;
   a.E = (int)E;
+  if (E <= mlxq::kStripRunsMax) {
+    // A run is dealt out past 3/4 of the passes that a CU has to do in all (a
+    // run of that length keeps its workgroups as long as the rest keeps the
+    // CUs; 1/2 and 1 of them measured the same) and past two.  The workgroups
+    // that deal fill the CUs once, twice where two fit one (64 weight rows, up
+    // to 48 rows a pass).
+    const int cus = device_info(current_device()).cus;
+    const double per_cu = ((double)B / (16 * p.mt) + 0.5 * (double)E) * p.row_blocks / cus;
+    a.long_run = (int)(16 * p.mt * std::max(2.0, 0.75 * per_cu));
+    a.deal = (int)std::min<int64_t>(E, std::max<int64_t>(1, (p.nwn == 4 && p.mt <= 3 ? 2 : 1) * (int64_t)cus / p.row_blocks));
+  }
   a.w_expert_stride = View{w}.dim(-2) * View{w}.dim(-1);
   a.s_expert_stride = View{scales}.dim(-2) * View{scales}.dim(-1);
   hip_check(mlxq::strip_launch(fmt, sp.bits, a, p, stream), "gather strip launch");

@@ -352,6 +352,7 @@ struct StripArgs {
   int M, N, K, gs_shift;
   int xt;                  // 16-bit type: 0 bfloat16, 1 float16
   int E;                   // experts (gathers)
+  int long_run, deal;      // gathers: past a run of this many entries, the workgroup rows that deal out all passes (0: never; E <= kStripRunsMax)
   int64_t w_expert_stride; // words per expert
   int64_t s_expert_stride; // scales per expert
   int ks, k_per_split;     // K ranges (dense), set by strip_launch
@@ -359,6 +360,7 @@ struct StripArgs {
 // 128-position windows per wave and staged step (LDS holds two steps of
 // activations; longer steps mean fewer barriers)
 constexpr int strip_wps(int mt, int nwn) { return mt == 1 && nwn >= 2 ? 2 : 1; }
+constexpr int kStripRunsMax = 512;  // experts whose runs a workgroup keeps, one per thread
 struct StripPlan {
   bool ok = false;
   int mt = 1;              // 16-row activation tiles per pass

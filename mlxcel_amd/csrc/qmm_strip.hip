@@ -9,9 +9,10 @@ namespace mlxq {
 
 namespace {
 
-size_t strip_lds(int mt, int nwn, int gs) {
+size_t strip_lds(int mt, int nwn, int gs, int64_t experts) {
   const int sr = (8 / nwn) * 128 * strip_wps(mt, nwn);
-  return (size_t)2 * mt * 16 * sr * 2 + (size_t)2 * (sr / gs) * (16 * nwn + 16) * 4 + 16;
+  return (size_t)2 * mt * 16 * sr * 2 + (size_t)2 * (sr / gs) * (16 * nwn + 16) * 4 + 16 +
+         (experts > 0 && experts <= kStripRunsMax ? (size_t)(2 * experts + 9) * 4 : 0);
 }
 
 // Microseconds of a launch on MI355X: start + per-window time of a wave
@@ -47,7 +48,7 @@ StripPlan strip_plan(int fmt, int bits, int gs, int64_t rows, int64_t N, int64_t
     const int nwn = 1 << ln;
     if (kWindow[lm][ln] == 0.f || (nwn_req > 0 && nwn != nwn_req)) continue;
     const int wps = strip_wps(mt, nwn), sr = (8 / nwn) * 128 * wps;
-    if (sr < 2 * gs || strip_lds(mt, nwn, gs) > kQmvLdsMax) continue;
+    if (sr < 2 * gs || strip_lds(mt, nwn, gs, experts) > kQmvLdsMax) continue;
     const int64_t blocks = (N + 16 * nwn - 1) / (16 * nwn);
     const int64_t steps = (K + sr - 1) / sr;
     const int64_t ks_max = experts > 0 ? 1 : ks_req > 0 ? ks_req : std::min<int64_t>(16, std::max<int64_t>(1, cus / blocks));
@@ -72,7 +73,7 @@ StripPlan strip_plan(int fmt, int bits, int gs, int64_t rows, int64_t N, int64_t
       p.ks = (int)ksr;
       p.k_per_split = (int)std::min<int64_t>(per_split * sr, (int64_t)1 << 30);
       p.windows = (int)windows;
-      p.lds = strip_lds(mt, nwn, gs);
+      p.lds = strip_lds(mt, nwn, gs, experts);
     }
   }
   if (p.ok && (p.row_blocks * (int64_t)16 * p.nwn >= ((int64_t)1 << 31) || p.ks > 65535 || experts > 65535)) p.ok = false;
@@ -85,6 +86,10 @@ hipError_t strip_launch(int fmt, int bits, const StripArgs& a_in, const StripPla
   a.ks = p.ks;
   a.k_per_split = p.k_per_split;
   const dim3 grid((unsigned)p.row_blocks, (unsigned)(a.rhs ? a.E : p.ks));
+  if (a.rhs) {  // bfloat16 4- and 8-bit codes only
+    if (fmt == MXFP4 || a.xt != 0 || (bits != 4 && bits != 8)) return hipErrorInvalidValue;
+    return bits == 4 ? strip_launch_fmt<AFF4, 4, 0, true>(a, p, grid, stream) : strip_launch_fmt<AFF4, 8, 0, true>(a, p, grid, stream);
+  }
   if (fmt == MXFP4) return a.xt == 0 ? strip_launch_fmt<MXFP4, 4, 0>(a, p, grid, stream) : hipErrorInvalidValue;
   if (bits == 4 || bits == 8) {
     if (a.xt != 0) return strip_launch_f16(bits, a, p, grid, stream);

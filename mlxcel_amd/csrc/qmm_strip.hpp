@@ -33,8 +33,14 @@
 // 4 windows and rings of 2 to 8; two workgroups per CU instead of one
 // changed nothing.
 //
-// Gathers sorted by expert (a.rhs): blockIdx.y is the expert, whose entries
-// are found by binary search in the sorted indices and taken 16 MT at a time.
+// Gathers sorted by expert (GATHER): workgroup row y takes expert y, whose
+// entries are found by binary search in the sorted indices, 16 MT of them at
+// a pass.  Routing that sends much of a batch to a few experts would leave
+// their passes to a few workgroups: where one run exceeds a.long_run entries,
+// the first a.deal workgroup rows find all runs (strip_runs) and deal the
+// passes of all experts out in turn (128 experts of 768 x 2048, 1024 tokens
+// top 8 all on the same 8 experts: 309 us without, 82 with; spread evenly 107
+// either way).
 
 #pragma once
 
@@ -57,7 +63,55 @@ __device__ __forceinline__ uint32_t strip_pack(float lo, float hi) {
   }
 }
 
-template <int FMT, int BITS, int XT, int MT, int NWN>
+// Sorted gathers whose longest run is far above the average: every expert's
+// entries, found by scanning the indices.  Expert e's run from `at[e]` to
+// `at[e + 1]` goes in passes of ROWS entries, the first of them number
+// `pass0[e]`; returns the number of passes.  (Called by all 512 threads, E <=
+// 512; at: E + 1 words, pass0: E + 8.)  Indices that are not sorted give runs
+// that overlap or lack entries, within [0, M].
+template <int ROWS>
+__device__ __forceinline__ int strip_runs(const StripArgs& a, int t, int* at, int* pass0) {
+  const int E = a.E, M = a.M, st = a.rhs_stride > 1 ? 2 : 1;
+  for (int e = t; e <= E; e += 512) at[e] = M;
+  __syncthreads();
+  for (int i0 = t; i0 < M; i0 += 512 * 8) {  // 16 loads in flight
+    uint32_t cur[8], prev[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      const int i = i0 + 512 * u;
+      cur[u] = a.rhs[(uint32_t)(min(i, M - 1) * st)];
+      prev[u] = a.rhs[(uint32_t)(max(min(i, M) - 1, 0) * st)];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      const int i = i0 + 512 * u;
+      if (i >= M) break;
+      const int c = (int)min(cur[u], (uint32_t)(E - 1)), p = i > 0 ? (int)min(prev[u], (uint32_t)(E - 1)) : -1;
+      for (int e = p + 1; e <= c; e++) at[e] = i;  // the first entry of every expert up to c
+    }
+  }
+  __syncthreads();
+  const int own = t < E ? (max(0, at[t + 1] - at[t]) + ROWS - 1) / ROWS : 0, lane = t & 63;
+  int sum = own;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int v = __shfl_up(sum, d);
+    if (lane >= d) sum += v;
+  }
+  if (lane == 63) pass0[E + (t >> 6)] = sum;
+  __syncthreads();
+  int before = sum - own, all = 0;
+#pragma unroll
+  for (int w = 0; w < 8; w++) {
+    const int v = pass0[E + w];
+    all += v;
+    if (w < (t >> 6)) before += v;
+  }
+  if (t < E) pass0[t] = before;
+  return all;
+}
+
+template <int FMT, int BITS, int XT, int MT, int NWN, bool GATHER>
 __global__ __launch_bounds__(512, 2) void qmm_strip_kernel(const StripArgs a) {
   constexpr bool AFF = FMT != MXFP4;
   constexpr int WPS = strip_wps(MT, NWN);    // windows per wave and step
@@ -93,32 +147,66 @@ __global__ __launch_bounds__(512, 2) void qmm_strip_kernel(const StripArgs a) {
   const int N = a.N, K = a.K;
   const int n0 = blockIdx.x * RW;
 
+  // gathers: workgroup y takes expert y's run of entries; where some run is
+  // far above the average, passes y, y + deal, ... of all experts' instead
   int first = 0, end = a.M;
-  int64_t wbase = 0, sbase = 0;
-  if (a.rhs) {
-    const int e = blockIdx.y;
-    sorted_run(a.rhs, a.rhs_stride, a.M, a.E, e, lane, first, end);
-    if (first >= end) return;  // the same in every wave
-    wbase = (int64_t)e * a.w_expert_stride;
-    sbase = (int64_t)e * a.s_expert_stride;
+  int64_t e = 0;
+  bool even = true;
+  int passes = 0;
+  volatile int* turn = reinterpret_cast<volatile int*>(big + 1);  // expert, first entry and end of a pass
+  int* at = reinterpret_cast<int*>(tbl + 2 * GS * TP) + 4;        // E + 1 words
+  int* pass0 = at + a.E + 1;                                      // E + 8
+  auto take = [&](int pass) {
+    __syncthreads();  // pass0 is written, the last turn read
+    if (t < a.E) {
+      const int i = (pass - pass0[t]) * (16 * MT), from = at[t], to = at[t + 1];
+      if (i >= 0 && from + i < to) {  // one thread's
+        turn[0] = t;
+        turn[1] = from + i;
+        turn[2] = min(to, from + i + 16 * MT);
+      }
+    }
+    __syncthreads();
+    e = __builtin_amdgcn_readfirstlane(turn[0]);
+    first = __builtin_amdgcn_readfirstlane(turn[1]);
+    end = __builtin_amdgcn_readfirstlane(turn[2]);
+  };
+  if constexpr (GATHER) {
+    e = blockIdx.y;
+    // A run longer than long_run + half covers some pair of entries long_run
+    // apart that starts at a multiple of half.  Every wave looks for itself
+    // (64 pairs a time, in flight beside the search): no barrier, and the same
+    // answer in all.
+    const int half = (a.long_run + 1) / 2, st = a.rhs_stride > 1 ? 2 : 1;
+    auto pair_at = [&](int i, uint32_t* v) {  // (past the end: one entry twice, masked by equal)
+      v[0] = a.rhs[(uint32_t)(min(i, a.M - 1) * st)];
+      v[1] = a.rhs[(uint32_t)(min(i + a.long_run, a.M - 1) * st)];
+    };
+    auto equal = [&](int i, const uint32_t* v) { return a.long_run > 0 && i + a.long_run < a.M && v[0] == v[1]; };
+    uint32_t v0[2];
+    sorted_run(a.rhs, a.rhs_stride, a.M, a.E, (int)e, lane, first, end, [&] { pair_at(lane * half, v0); });
+    even = __ballot(equal(lane * half, v0)) == 0ull;
+    for (int i = (64 + lane) * half; even && a.long_run > 0 && (i - lane * half) + a.long_run < a.M; i += 64 * half) {
+      uint32_t v[2];
+      pair_at(i, v);
+      even = __ballot(equal(i, v)) == 0ull;
+    }
+    if (even) {
+      if (first >= end) return;  // the same in every wave
+    } else {
+      if ((int)blockIdx.y >= a.deal) return;
+      passes = __builtin_amdgcn_readfirstlane(strip_runs<16 * MT>(a, t, at, pass0));
+      if ((int)blockIdx.y >= passes) return;
+      take(blockIdx.y);
+    }
   }
-  const int z = a.rhs ? 0 : blockIdx.y;
+  const int z = GATHER ? 0 : blockIdx.y;
   const int kbeg = z * a.k_per_split, kend = min(K, kbeg + a.k_per_split);
   const int nsteps = (kend - kbeg + SR - 1) / SR;
 
   const int G = K >> gs_shift;
   const uint32_t RB = (uint32_t)(K / 32 * BITS) * 4u;
   constexpr uint32_t SE = AFF ? 2u : 1u;     // bytes per scale
-  const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(a.x, (uint32_t)((int64_t)a.M * K * 2));
-  const __amdgpu_buffer_rsrc_t wr = buffer_rsrc(a.w + wbase, (uint32_t)((int64_t)N * RB));
-  const __amdgpu_buffer_rsrc_t sr =
-      buffer_rsrc(static_cast<const uint8_t*>(a.scales) + sbase * SE, (uint32_t)((int64_t)N * G * SE));
-  const __amdgpu_buffer_rsrc_t br =
-      buffer_rsrc(AFF ? (const void*)(static_cast<const uint8_t*>(a.biases) + sbase * SE) : a.scales,
-                  AFF ? (uint32_t)((int64_t)N * G * SE) : 0u);
-
-  // empty resources for the loads of steps past the end
-  const __amdgpu_buffer_rsrc_t x0 = buffer_rsrc(a.x, 0u), w0 = buffer_rsrc(a.w, 0u), s0r = buffer_rsrc(a.scales, 0u);
 
   // weights of this lane: row n0 + 16 nwave + r, codes 32 q .. + 31 of each
   // window; positions past K read the next row's codes (finite, and their
@@ -126,10 +214,6 @@ __global__ __launch_bounds__(512, 2) void qmm_strip_kernel(const StripArgs a) {
   const int wn = n0 + 16 * nwave + r;
   const uint32_t woff = wn < N ? (uint32_t)wn * RB + (uint32_t)(((kbeg + kwave * SRW) >> 5) + q) * (uint32_t)(BITS * 4) : kDeadOfs;
   uint32_t wv[RD][BITS];
-  auto load_window = [&](int slot, int step, int w) {
-    const bool live = step < nsteps;
-    load_codes<BITS>(live ? wr : w0, woff, live ? (step * (SR / 32) + w * 4) * (BITS * 4) : 0, wv[slot]);
-  };
 
   // activations: thread t stages chunk t % CPR of rows t / CPR + XROWS i
   const int xrow = t / CPR, xch = t % CPR;
@@ -149,8 +233,22 @@ __global__ __launch_bounds__(512, 2) void qmm_strip_kernel(const StripArgs a) {
     soff[i] = row < RW && n < N ? ((uint32_t)n * (uint32_t)G + (uint32_t)g) * SE : kDeadOfs;
   }
 
-  for (int c0 = first; c0 < end; c0 += 16 * MT) {
+  const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(a.x, (uint32_t)((int64_t)a.M * K * 2));
+  // empty resources for the loads of steps past the end
+  const __amdgpu_buffer_rsrc_t x0 = buffer_rsrc(a.x, 0u), w0 = buffer_rsrc(a.w, 0u), s0r = buffer_rsrc(a.scales, 0u);
+  for (int c0 = first, pass = blockIdx.y;;) {
     const int rows = min(16 * MT, end - c0);
+    const int64_t sofs = e * a.s_expert_stride * SE;
+    const __amdgpu_buffer_rsrc_t wr = buffer_rsrc(a.w + e * a.w_expert_stride, (uint32_t)((int64_t)N * RB));
+    const __amdgpu_buffer_rsrc_t sr =
+        buffer_rsrc(static_cast<const uint8_t*>(a.scales) + sofs, (uint32_t)((int64_t)N * G * SE));
+    const __amdgpu_buffer_rsrc_t br =
+        buffer_rsrc(AFF ? (const void*)(static_cast<const uint8_t*>(a.biases) + sofs) : a.scales,
+                    AFF ? (uint32_t)((int64_t)N * G * SE) : 0u);
+    auto load_window = [&](int slot, int step, int w) {
+      const bool live = step < nsteps;
+      load_codes<BITS>(live ? wr : w0, woff, live ? (step * (SR / 32) + w * 4) * (BITS * 4) : 0, wv[slot]);
+    };
 #pragma unroll
     for (int i = 0; i < XL; i++) {
       const int row = xrow + XROWS * i;
@@ -363,14 +461,23 @@ __global__ __launch_bounds__(512, 2) void qmm_strip_kernel(const StripArgs a) {
       }
     }
     __syncthreads();  // the sums have been read before the next rows are staged
+    if (!GATHER || even) {
+      c0 += 16 * MT;
+      if (c0 >= end) break;
+    } else {
+      pass += a.deal;
+      if (pass >= passes) break;
+      take(pass);
+      c0 = first;
+    }
   }
 }
 
-template <int FMT, int BITS, int XT>
+template <int FMT, int BITS, int XT, bool GATHER = false>
 hipError_t strip_launch_fmt(const StripArgs& a, const StripPlan& p, dim3 grid, hipStream_t stream) {
 #define STRIP_CASE(MT_, NWN_)                                                                                      \
   if (p.mt == MT_ && p.nwn == NWN_) {                                                                              \
-    hipLaunchKernelGGL((qmm_strip_kernel<FMT, BITS, XT, MT_, NWN_>), grid, dim3(512), p.lds, stream, a);           \
+    hipLaunchKernelGGL((qmm_strip_kernel<FMT, BITS, XT, MT_, NWN_, GATHER>), grid, dim3(512), p.lds, stream, a);   \
     return hipGetLastError();                                                                                      \
   }
   STRIP_CASE(1, 1)

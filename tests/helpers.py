@@ -63,3 +63,41 @@ def mxfp4_case(M, N, K, seed, E=None):
     w = orc.normal_bf16(shape, 0.02, seed + 1)
     wq, s = orc.mxfp4_quantize(w)
     return x, wq, s
+
+
+def kernels_of(fn):
+    """Names of the GPU kernels that fn() launches."""
+    from torch.profiler import ProfilerActivity, profile
+
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        fn()
+        torch.cuda.synchronize()
+    return [e.name for e in p.events() if str(e.device_type).endswith("CUDA")]
+
+
+def graph_us(fns, reps=10):
+    """Microseconds per call of each function, their captured calls replayed in turn (medians)."""
+    s = torch.cuda.Stream()
+    graphs = []
+    for fn in fns:
+        with torch.cuda.stream(s):
+            fn()
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            for _ in range(reps):
+                fn()
+        graphs.append(g)
+    times = [[] for _ in fns]
+    with torch.cuda.stream(s):
+        for rep in range(8):
+            for t, g in zip(times, graphs):
+                a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                a.record()
+                g.replay()
+                b.record()
+                b.synchronize()
+                if rep:
+                    t.append(a.elapsed_time(b) * 1e3 / reps)
+    return [sorted(t)[len(t) // 2] for t in times]

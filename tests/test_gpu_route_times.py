@@ -1,0 +1,46 @@
+"""Calls whose default route must not be slower than another kernel of this
+library takes for them: each was once given a kernel 1.4 to 8 times slower.
+Both are timed here in turn (captured calls, medians); a quarter over is
+allowed."""
+import pytest
+import torch
+
+import mlxcel_amd as mq
+from helpers import announce, graph_us, kernels_of, setknob
+
+pytestmark = pytest.mark.gpu
+
+
+def _matrix(shape, K, bits, gs):
+    g = torch.Generator(device="cuda").manual_seed(7)
+    w = torch.randint(-2 ** 31, 2 ** 31, (*shape, K * bits // 32), generator=g, device="cuda").to(torch.int32)
+    s = torch.rand((*shape, K // gs), generator=g, device="cuda").to(torch.bfloat16) * 0.01
+    return w.view(torch.uint32), s, -8 * s
+
+
+def _timed(monkeypatch, call, other):
+    """(us of the default route, us with the switches of `other` set)"""
+    def switched():
+        with monkeypatch.context() as m:
+            for k, v in other.items():
+                setknob(m, k, v)
+            call()
+        setknob(monkeypatch, "MLXQ_NONE", "")  # re-read the switches
+
+    return graph_us([call, switched])
+
+
+@pytest.mark.parametrize("E,N,K,B,hot", [(128, 768, 2048, 8192, 8), (128, 768, 2048, 1024, 8), (32, 2048, 1024, 2048, 2)])
+def test_skewed_sorted_gather(monkeypatch, E, N, K, B, hot):
+    # all entries on a few experts, against the grouped tiles
+    announce("route time, skewed gather", E, N, K, B, hot)
+    w, s, b = _matrix((E, N), K, 4, 64)
+    x = torch.randn(B, 1, K, device="cuda").to(torch.bfloat16)
+    ids = (torch.arange(hot, device="cuda").repeat_interleave(B // hot) * (E // hot)).to(torch.int32)
+
+    def call():
+        return mq.gather_qmm(x, w, s, b, None, ids, True, 64, 4, "affine", True)
+
+    now, tiles = _timed(monkeypatch, call, {"MLXQ_STRIP": "0"})
+    assert any("qmm_strip" in k for k in kernels_of(call))
+    assert now <= 1.25 * tiles, (now, tiles)

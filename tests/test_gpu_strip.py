@@ -144,3 +144,35 @@ def test_rows_in_passes(bits, dt):
     (wq, s, b), (wqn, sv, bv) = _weights(rng, (N,), K, bits, gs, dt)
     y = mq.quantized_matmul(x, wq, s, b, True, gs, bits)
     assert _rel(y, og.qmm(xv, wqn, sv, bv, True, gs, bits), dt) <= 1e-2
+
+
+# counts of entries per expert: one long run among short ones, all on one
+# expert (the first, the last), several long runs, as many experts as a
+# workgroup keeps runs of (512) and one more
+LONG = {"one": [3, 0, 600, 1, 17, 0, 2, 9, 1, 0, 0, 5, 0, 1, 0, 1], "first": [512] + [0] * 7, "last": [0] * 7 + [513],
+        "two": [0] * 20 + [700] + [1] * 20 + [900] + [2] * 22, "512": [8, 700] * 4 + [3] * 504, "513": [8, 700] * 4 + [3] * 505}
+
+
+@pytest.mark.parametrize("bits,gs,K", [(4, 64, 192), (8, 64, 320)])
+@pytest.mark.parametrize("mt", [1, 2, 3, 8])
+@pytest.mark.parametrize("name", sorted(LONG))
+def test_sorted_gather_with_long_runs(monkeypatch, bits, gs, K, mt, name):
+    # runs far above the average are dealt out over the workgroups
+    setknob(monkeypatch, "MLXQ_STRIP", "2")
+    setknob(monkeypatch, "MLXQ_STRIP_MT", str(mt))
+    counts = LONG[name]
+    E, N = len(counts), 68 if len(counts) > 64 else 200
+    rng = np.random.default_rng(45500 + bits + mt)
+    ids = np.repeat(np.arange(E), counts)
+    announce("strip gather long runs", bits, mt, name)
+    x, xv = _dev(rng.standard_normal((len(ids), 1, K)), "bfloat16")
+    (wq, s, b), (wqn, sv, bv) = _weights(rng, (E, N), K, bits, gs, "bfloat16")
+    want = np.concatenate([og.qmm(xv[ids == e, 0], wqn[e], sv[e], bv[e], True, gs, bits) for e in range(E) if counts[e]])
+    for idx in (torch.int32, torch.int64):
+        i = torch.from_numpy(ids).to(idx).cuda()
+        y = mq.gather_qmm(x, wq, s, b, None, i, True, gs, bits, "affine", True)
+        assert _rel(y[:, 0], want, "bfloat16") <= 1e-2
+        assert torch.equal(y, mq.gather_qmm(x, wq, s, b, None, i, True, gs, bits, "affine", True))
+    # indices past the experts belong to the last one
+    i = torch.from_numpy(np.where(ids == E - 1, E + 5 + np.arange(len(ids)), ids)).to(torch.int32).cuda()
+    assert torch.equal(y, mq.gather_qmm(x, wq, s, b, None, i, True, gs, bits, "affine", True))
