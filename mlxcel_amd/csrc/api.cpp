@@ -1400,7 +1400,8 @@ bool try_strip(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, cons
   return true;
 }
 
-// Sorted gathers of affine codes with one row per entry and at least 8
+// Sorted gathers of the specialised kernels' affine calls (bfloat16, 4- or
+// 8-bit codes, transpose=true) with one row per entry and at least 8
 // entries per touched expert, where the kernels for grouped rows round the
 // weights too (fewer run the block-MFMA search kernel, which does not): a
 // workgroup per 64 weight rows of an expert finds the expert's entries in
@@ -1412,13 +1413,12 @@ bool try_strip_gather(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* 
                       const mlxq_array* biases, const DirectIdx& dl, const DirectIdx& dr, mlxq_array* out, int64_t B,
                       int64_t E, hipStream_t stream) {
   const Knobs& kn = knobs();
-  if (kn.strip == 0 || !strip_types(sp, x, scales, biases)) return false;
-  if (kn.strip != 2 && (sp.mode != AFFINE || !rounds_weights(sp) || kn.gather_group >= 0 || kn.gather_sorted == 0 || B < 8 * std::min(E, B)))
+  if (kn.strip == 0 || sp.mode != AFFINE || !biases) return false;
+  if (kn.strip != 2 && (!rounds_weights(sp) || kn.gather_group >= 0 || kn.gather_sorted == 0 || B < 8 * std::min(E, B)))
     return false;
   // one row of x per entry, indices read in place
   if (!dr.ok || !dr.p || !dl.ok || dl.p || dl.div != 1) return false;
-  const int fmt = sp.mode == MXFP4_M ? mlxq::MXFP4 : mlxq::AFF4;
-  const mlxq::StripPlan p = mlxq::strip_plan(fmt, sp.bits, sp.gs, B, sp.N, sp.K, E, device_info(current_device()).cus,
+  const mlxq::StripPlan p = mlxq::strip_plan(mlxq::AFF4, sp.bits, sp.gs, B, sp.N, sp.K, E, device_info(current_device()).cus,
                                              kn.strip_nwn, kn.strip_mt, 0);
   if (!p.ok) return false;
   // many rows for few workgroups: the passes of 128 rows run one after the
@@ -1429,9 +1429,8 @@ bool try_strip_gather(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* 
   a.x = static_cast<const uint16_t*>(x->data);
   a.w = static_cast<const uint32_t*>(w->data);
   a.scales = scales->data;
-  a.biases = biases ? biases->data : nullptr;
+  a.biases = biases->data;
   a.out = static_cast<uint16_t*>(out->data);
-  a.xt = sp.out_dtype == MLXQ_FLOAT16 ? 1 : 0;
   a.M = (int)B;
   a.N = (int)sp.N;
   a.K = (int)sp.K;
@@ -1452,7 +1451,7 @@ bool try_strip_gather(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* 
   }
   a.w_expert_stride = View{w}.dim(-2) * View{w}.dim(-1);
   a.s_expert_stride = View{scales}.dim(-2) * View{scales}.dim(-1);
-  hip_check(mlxq::strip_launch(fmt, sp.bits, a, p, stream), "gather strip launch");
+  hip_check(mlxq::strip_launch(mlxq::AFF4, sp.bits, a, p, stream), "gather strip launch");
   return true;
 }
 
