@@ -16,7 +16,7 @@ import torch
 
 import mlxcel_amd as mq
 from oracle import generic as og
-from helpers import announce, dev_u32, setknob
+from helpers import announce, dev_u32, kernels_of, setknob
 
 pytestmark = pytest.mark.gpu
 
@@ -144,6 +144,26 @@ def test_rows_in_passes(bits, dt):
     (wq, s, b), (wqn, sv, bv) = _weights(rng, (N,), K, bits, gs, dt)
     y = mq.quantized_matmul(x, wq, s, b, True, gs, bits)
     assert _rel(y, og.qmm(xv, wqn, sv, bv, True, gs, bits), dt) <= 1e-2
+
+
+@pytest.mark.parametrize("bits,gs,K", [(8, 64, 320), (8, 32, 192), (8, 128, 640), (4, 64, 320)])
+@pytest.mark.parametrize("counts", [[110, 128, 120], [140, 1, 129, 0, 260], [16, 40, 1, 0, 33, 16], [8, 9, 10, 11]])
+def test_sorted_gather_runs_here(monkeypatch, bits, gs, K, counts):
+    # 8-bit codes, and passes of 128 rows with tails; forced, so that no other
+    # kernel can stand in
+    setknob(monkeypatch, "MLXQ_STRIP", "2")
+    rng = np.random.default_rng(45300 + bits + sum(counts))
+    E, N = len(counts), 100
+    ids = np.repeat(np.arange(E), counts)
+    announce("strip gather forced", bits, gs, counts)
+    x, xv = _dev(rng.standard_normal((len(ids), 1, K)), "bfloat16")
+    (wq, s, b), (wqn, sv, bv) = _weights(rng, (E, N), K, bits, gs, "bfloat16")
+    i = torch.from_numpy(ids).cuda()
+    out = []
+    names = kernels_of(lambda: out.append(mq.gather_qmm(x, wq, s, b, None, i, True, gs, bits, "affine", True)))
+    assert len(names) == 1 and "qmm_strip" in names[0], names
+    want = np.stack([og.qmm(xv[i], wqn[e], sv[e], bv[e], True, gs, bits) for i, e in enumerate(ids)])
+    assert _rel(out[0], want, "bfloat16") <= 1e-2
 
 
 # counts of entries per expert: one long run among short ones, all on one
