@@ -1311,6 +1311,13 @@ bool try_qmm_tile(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, c
   const mlxq::QmmPlan qp = prefill_plan(fmt, sp.gs, rows, sp.N, sp.K, dev, stream, ss, tile_req, knobs().qmm_ksplit,
                                         knobs().qmm_mix, knobs().qmm_streamk, &cnt);
   if (!qp.ok || qp.tile < 4) return false;
+  // small matrices: the general kernel where it is priced lower (3-bit 257
+  // rows over 155 x 1024 10.4 us vs 17.3, 2-bit 488 rows over 282 x 512 11.4 vs
+  // 16.6, 5-bit 316 rows over 153 x 1152 12.5 vs 17.6)
+  if (odd && tile_req < 0 && knobs().qmm_ksplit <= 0) {
+    const int cus = device_info(dev).cus;
+    if (mlxq::gen_us(mlxq::gen_plan(rows, sp.N, sp.K, 1, cus, 0), rows, sp.N, cus) < qp.us) return false;
+  }
   mlxq::QmmArgs q{};
   q.x = static_cast<const uint16_t*>(x->data);
   q.w = static_cast<const uint32_t*>(w->data);
@@ -1375,10 +1382,22 @@ bool try_strip(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, cons
   const int fmt = sp.mode == MXFP4_M ? mlxq::MXFP4 : mlxq::AFF4;
   mlxq::StripPlan p = mlxq::strip_plan(fmt, sp.bits, sp.gs, rows, sp.N, sp.K, 0, cus, kn.strip_nwn, kn.strip_mt, kn.strip_ks);
   if (!p.ok || (!forced && !odd && rows > 64 && p.windows > 4)) return false;
-  // several passes only where they fill half the CUs (6-bit, 512 rows: 4096 x
-  // 4128 91 us vs 267 on the general kernel; 1000 rows over 1100 x 544, 54
-  // workgroups, 85 vs 28)
-  if (!forced && rows > 128 && (int64_t)p.row_blocks * p.ks * 2 < cus) return false;
+  if (!forced) {
+    // where the kernels below are priced lower they keep the call: the general
+    // kernel many rows and small matrices (6-bit 1000 rows over 1100 x 544 28 us
+    // vs 85, 5-bit 739 rows over 5645 x 544 44 vs 79, 98 rows over 169 x 1024
+    // 10.7 vs 13.9), the prefill tiles many rounds with a short K (4-bit 78 rows
+    // over 151936 x 256 27 vs 80, 52 rows 26 vs 49; 8-bit 49 rows over 151936 x
+    // 1152 72 vs 114).  Of 3100 timed calls at 5-128 rows 9 are more than 5%
+    // slower than on the other kernel.
+    const float other = odd ? mlxq::gen_us(mlxq::gen_plan(rows, sp.N, sp.K, 1, cus, 0), rows, sp.N, cus)
+                            : mlxq::qmm_plan(fmt_of(sp.mode, sp.bits), sp.gs, rows, sp.N, sp.K, cus, -1, 0).us;
+    if (other > 0.f && p.us > other) return false;
+    // mxfp4 rows that the tiles do not take (K not a multiple of 64) have the
+    // skinny kernel, 9.6-11 us for up to 128 rows of small matrices where one
+    // pass of strips takes 12
+    if (sp.mode == MXFP4_M && sp.K % 64 != 0 && rows > 72 && sp.K < 1664 && sp.N <= 640) return false;
+  }
   auto part = [&] { return (size_t)p.ks * rows * sp.N * sizeof(float); };
   // partials that cannot be had here: the kernels below
   if (p.ks > 1 && !scratch_fits(dev, stream, part(), ss)) return false;

@@ -150,6 +150,9 @@ struct GenPlan {
 };
 // ks_req > 0 forces the K split (tests)
 GenPlan gen_plan(int64_t M, int64_t N, int64_t K, int64_t nseg, int cus, int ks_req);
+// microseconds of that plan for 5 rows and more of 2-, 3-, 5- or 6-bit codes,
+// 16-bit types, transpose=true
+float gen_us(const GenPlan& p, int64_t M, int64_t N, int cus);
 // tc: GenType of the MFMA inputs and of `out`
 hipError_t qmm_gen_launch(const GenArgs& a, const GenPlan& p, int tc, bool transpose, int64_t nseg,
                           hipStream_t stream);
@@ -367,6 +370,7 @@ struct StripPlan {
   int nwn = 4;             // waves along the weight rows (16 rows each)
   int row_blocks = 0, ks = 1, k_per_split = 0;
   int windows = 0;         // 128-position windows each wave multiplies
+  float us = 0.f;          // price of a dense launch
   size_t lds = 0;
 };
 StripPlan strip_plan(int fmt, int bits, int gs, int64_t rows, int64_t N, int64_t K, int64_t experts, int cus,
@@ -445,6 +449,7 @@ struct QmmPlan {
   int tile2 = -1, n_first = 0, tiles_n2 = 0;
   // Stream-K (sk_len > 0): sk_wgs workgroups of sk_len K-steps each.
   int sk_len = 0, sk_wgs = 0;
+  float us = 0.f;  // its price in one launch (0: none known)
 };
 // Counter words and fp32 partial bytes a stream-K plan needs.
 inline int64_t qmm_sk_counters(const QmmPlan& p) { return p.sk_len > 0 ? p.sk_wgs : 0; }

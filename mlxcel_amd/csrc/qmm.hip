@@ -246,6 +246,37 @@ bool is_tile_kernel(int tile) { return tile >= 4; }
 int qmm_tile_rows(int tile) { return tile >= 0 && tile < kTiles ? kBM[tile] : 0; }
 
 namespace {
+// Microseconds of a launch of tiles 4, 6 and 8 on MI355X:
+//   start + rounds * (round + K-steps * (step + step_fill * fill)) + partial sums
+// fill: workgroups over what one round of the CUs holds, at most 1; rounds: 1,
+// or the exact number of them, `whole` of the way to the next integer (part-full
+// rounds of one tile per CU cost more than a full one); a round's own
+// time grows with the fill and is longer where rows of the result cannot be
+// written 16 bytes at a time.  Fitted to 280000 graph-timed launches (129-2048
+// rows; 17-128 rows for `few`; N 64-151936, K 256-14336, half of them with N
+// not a multiple of 8), 5-6% rms.
+struct TileCost {
+  int slots;  // workgroups per CU
+  float start, round[2], round_fill[2], step, step_fill, whole, sum, sum_each;  // [0] 16-byte rows of the result, [1] others
+};
+constexpr TileCost kCost4 = {1, 0.1f, {4.3f, 9.9f}, {7.4f, 13.3f}, 0.86f, 0.65f, 1.71f, 4.8f, 0.95f};
+constexpr TileCost kCost6 = {2, 3.3f, {2.1f, 6.1f}, {4.1f, 6.4f}, 0.81f, 0.34f, 0.54f, 3.3f, 1.43f};
+constexpr TileCost kCost8 = {1, 3.4f, {1.8f, 5.8f}, {3.9f, 5.8f}, 0.78f, 0.23f, 1.28f, 3.6f, 1.49f};
+constexpr TileCost kCost6Few = {2, 0.8f, {4.4f, 6.4f}, {0.9f, 1.5f}, 0.81f, 0.40f, 0.51f, 3.0f, 2.23f};
+constexpr TileCost kCost4Odd = {1, 3.7f, {2.6f, 8.8f}, {6.4f, 12.4f}, 1.01f, 0.65f, 1.57f, 4.9f, 0.91f};
+constexpr TileCost kCost6Odd = {2, 4.3f, {1.2f, 5.0f}, {4.2f, 6.8f}, 0.86f, 0.38f, 0.54f, 3.2f, 1.38f};
+
+float tile_us(int tile, bool odd, int64_t M, int64_t N, int nks, int ks, int num_cus) {
+  const TileCost& c = tile == 4 ? (odd ? kCost4Odd : kCost4) : tile == 8 ? kCost8 : odd ? kCost6Odd : M <= 128 ? kCost6Few : kCost6;
+  const int steps = (nks + ks - 1) / ks, ksr = (nks + steps - 1) / steps;
+  const int64_t tiles = ((M + kBM[tile] - 1) / kBM[tile]) * ((N + kBN[tile] - 1) / kBN[tile]);
+  const float x = (float)(tiles * ksr) / (float)((int64_t)c.slots * num_cus), fill = std::min(x, 1.f);
+  const float rounds = std::max(1.f, c.whole * std::ceil(x) + (1.f - c.whole) * x);
+  const int narrow = N % (ksr > 1 ? 4 : 8) != 0;
+  return c.start + rounds * (c.round[narrow] + c.round_fill[narrow] * fill + steps * (c.step + c.step_fill * fill)) +
+         (ksr > 1 ? c.sum + c.sum_each * (float)ksr * M * N * 1e-6f : 0.f);
+}
+
 // Tile and K split of a grid that fits about one round of the CUs (129-1024
 // rows; the 2-, 3-, 5- and 6-bit codes, which have no 256 x 128 tile on 8
 // waves, at any row count).  One round of 256 x 128 tiles (3/4 to all of the
@@ -302,10 +333,20 @@ QmmPlan qmm_plan(int fmt, int gs, int64_t M, int64_t N, int64_t K, int num_cus, 
   const int nks = (int)(K / BK);
   auto tiles_of = [&](int t) { return ((M + kBM[t] - 1) / kBM[t]) * ((N + kBN[t] - 1) / kBN[t]); };
   int tile, ks_planned = 0;
+  // K split by powers of two while the grid covers less than the CUs (up to
+  // two workgroups per CU for few rows, where each tile is cheap) and each
+  // split keeps >= 8 K-steps (gate/up M=32-128: 448 workgroups 31-38 us, 896
+  // 37-50 us)
+  auto pow2_split = [&](int t) {
+    const int64_t n = tiles_of(t), fit = M <= 128 ? 2 * (int64_t)num_cus : num_cus;
+    int ks = 1;
+    while (n * ks * 2 <= fit && nks / (ks * 2) >= 8) ks *= 2;
+    return ks;
+  };
   if (tile_req >= 0 && tile_req < kTiles) {
     tile = tile_req;
-  } else if (fit_round && (odd || (M > 128 && M <= 1024 && tiles_of(4) <= num_cus))) {
-    tile = plan_mid(odd, M, N, nks, num_cus, ks_planned);
+  } else if (odd) {
+    tile = plan_mid(true, M, N, nks, num_cus, ks_planned);
   } else {
     // 256 x 256 (8 waves) when there are enough tiles or K is long enough
     // for a K split to fill the CUs; else 128 x 128, two workgroups per CU.
@@ -323,33 +364,22 @@ QmmPlan qmm_plan(int fmt, int gs, int64_t M, int64_t N, int64_t K, int num_cus, 
     const bool one_round8 = (fmt == AFF8 && t8 * 4 >= (int64_t)num_cus * 3) || (fmt != MXFP4 && t8 <= num_cus);
     if (mid_rows && (K >= 8192 || one_round8)) tile = 8;
     else tile = (M > 128 && (tiles_of(4) >= num_cus / 2 || K >= 8192)) ? 4 : 6;
+    if (fit_round && ksplit_req <= 0 && M > 128 && M <= 1024 && tiles_of(4) <= num_cus)
+      tile = plan_mid(false, M, N, nks, num_cus, ks_planned);
   }
   p.tile = tile;
   p.rows_per_tile = kBM[tile];
   p.tiles_n = (int)((N + kBN[tile] - 1) / kBN[tile]);
   p.tiles_m = (int)((M + kBM[tile] - 1) / kBM[tile]);
   const int64_t tiles = (int64_t)p.tiles_n * p.tiles_m;
-  int ks = 1;
-  if (ksplit_req > 0) {
-    ks = ksplit_req;
-  } else if (ks_planned > 0) {
-    ks = ks_planned;
-  } else {
-    // split K while the grid covers less than the CUs (up to two workgroups
-    // per CU for few rows, where each tile is cheap) and each split keeps >= 8
-    // K-steps (gate/up M=32-128: 448 workgroups 31-38 us, 896 37-50 us)
-    if (M <= 128) {
-      while (tiles * ks * 2 <= 2 * num_cus && nks / (ks * 2) >= 8) ks *= 2;
-    } else {
-      while (tiles * ks * 2 <= num_cus && nks / (ks * 2) >= 8) ks *= 2;
-    }
-  }
+  const int ks = ksplit_req > 0 ? ksplit_req : ks_planned > 0 ? ks_planned : pow2_split(tile);
   p.ksteps_per_split = (nks + ks - 1) / ks;
   p.ksplit = (nks + p.ksteps_per_split - 1) / p.ksteps_per_split;
   // consecutive tiles along M share weights, along N share activations: walk
   // along the dimension whose operand is the smaller of the two to re-read
   p.m_fast = M * K * 2 <= N * K * bits / 8 ? 1 : 0;
   p.ok = tiles * p.ksplit < ((int64_t)1 << 31);
+  if (tile == 4 || tile == 6 || tile == 8) p.us = tile_us(tile, odd, M, N, nks, ks, num_cus);
   // Part-full last round: more 256 x 256 tiles than CUs, and the columns
   // past the whole rounds fit one round of 256 x 128 tiles.  Whole columns
   // of 256 x 256 tiles fill the full rounds, the rest runs as that one round

@@ -33,6 +33,9 @@
 // codes.
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
+#include <cmath>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -571,6 +574,21 @@ GenPlan gen_plan(int64_t M, int64_t N, int64_t K, int64_t nseg, int cus, int ks_
   p.ks = (ksteps + p.ksteps_per_split - 1) / p.ksteps_per_split;
   p.ok = (int64_t)p.tiles_m * p.ks <= 65535 && nseg <= 65535 && p.tiles_n <= (1 << 30);
   return p;
+}
+
+// Priced as the prefill tiles are (qmm.hip); fitted to 27600 graph-timed calls
+// on MI355X (5-2048 rows, N 64-20000, K 256-14336), 10% rms.
+float gen_us(const GenPlan& p, int64_t M, int64_t N, int cus) {
+  struct Cost {
+    int slots;  // workgroups per CU
+    float start, step, step_fill, whole, sum, sum_each, narrow;
+  };
+  constexpr Cost few = {4, 2.0f, 1.30f, 0.83f, 0.47f, 2.0f, 2.9f, 0.1f}, many = {6, 3.3f, 1.32f, 1.22f, 0.41f, 1.5f, 2.6f, 0.3f};
+  const Cost& c = p.bm == 16 ? few : many;
+  const float x = (float)((int64_t)p.tiles_m * p.tiles_n * p.ks) / (float)((int64_t)c.slots * cus), fill = std::min(x, 1.f);
+  const float rounds = std::max(1.f, c.whole * std::ceil(x) + (1.f - c.whole) * x);
+  return c.start + rounds * p.ksteps_per_split * (c.step + c.step_fill * fill) +
+         (p.ks > 1 ? c.sum + c.sum_each * (float)p.ks * M * N * 1e-6f : 0.f) + (N % 8 != 0 ? c.narrow : 0.f);
 }
 
 hipError_t qmm_gen_launch(const GenArgs& a0, const GenPlan& p, int tc, bool transpose, int64_t nseg,

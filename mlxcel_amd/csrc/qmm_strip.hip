@@ -15,12 +15,26 @@ size_t strip_lds(int mt, int nwn, int gs, int64_t experts) {
          (experts > 0 && experts <= kStripRunsMax ? (size_t)(2 * experts + 9) * 4 : 0);
 }
 
-// Microseconds of a launch on MI355X: start + per-window time of a wave
-// (fitted to graph-timed 4-bit g64 calls over 11 shapes from 1024 x 4096 to
-// 28672 x 4096; 3- and 6-bit codes lie within 15%), [kTilesM index][log2(nwn)].
 constexpr int kTilesM[5] = {1, 2, 3, 4, 8};  // 16-row activation tiles per pass
-constexpr float kStart[5][3] = {{4.0f, 5.0f, 3.6f}, {4.7f, 4.1f, 3.2f}, {0.f, 4.5f, 3.5f}, {0.f, 4.9f, 3.9f}, {0.f, 0.f, 4.2f}};
-constexpr float kWindow[5][3] = {{1.0f, 0.65f, 0.70f}, {1.3f, 1.1f, 0.98f}, {0.f, 1.32f, 1.10f}, {0.f, 1.53f, 1.21f}, {0.f, 0.f, 2.4f}};
+// Microseconds of a dense launch on MI355X:
+//   start + rounds * passes * (pass + window * windows of a wave) + partial sums
+// a pass is longer the fuller the round and where rows of the result cannot
+// be written 16 bytes at a time; rounds of workgroups past one count `whole`
+// of the way to the next integer (14336 x 4096 in 448 workgroups of 32 rows
+// 19.5 us, 8192 x 4096 in 256 of them 10.6).  Fitted to 80000 graph-timed
+// launches (5-128 rows, and passes of 128 to 1024; N 64-151936, K 256-14336),
+// 4-11% rms; [kTilesM index][log2(nwn)], window 0: not built.
+struct StripCost {
+  float start, pass, pass_fill, narrow, window, whole, sum, sum_each;
+};
+constexpr StripCost kCost[5][3] = {
+    {{3.6f, 0.4f, 0.4f, 0.6f, 0.94f, 0.64f, 2.3f, 13.9f}, {2.3f, 1.8f, 0.7f, 0.6f, 0.73f, 0.97f, 2.4f, 11.0f}, {3.6f, 0.0f, 0.9f, 0.6f, 0.64f, 0.78f, 2.7f, 1.8f}},
+    {{1.9f, 2.6f, 0.5f, 0.6f, 1.38f, 0.93f, 2.2f, 9.5f}, {2.1f, 1.8f, 0.6f, 0.6f, 1.02f, 0.83f, 2.4f, 4.8f}, {3.4f, 0.0f, 0.8f, 0.7f, 0.82f, 0.60f, 2.8f, 2.3f}},
+    {{}, {1.8f, 2.4f, 0.7f, 0.7f, 1.32f, 0.94f, 2.3f, 4.7f}, {3.7f, 0.0f, 0.8f, 0.9f, 1.05f, 0.67f, 2.5f, 3.7f}},
+    {{}, {1.9f, 2.7f, 0.9f, 0.7f, 1.49f, 0.95f, 2.3f, 3.8f}, {1.9f, 1.9f, 1.3f, 1.0f, 1.12f, 0.95f, 2.7f, 2.9f}},
+    {{}, {}, {1.5f, 2.9f, 1.5f, 2.3f, 1.84f, 0.96f, 2.8f, 2.3f}}};
+// the same by width of the codes
+constexpr float kBitsCost[9] = {1.f, 1.f, 0.97f, 0.99f, 0.97f, 1.04f, 1.03f, 1.f, 1.f};
 
 }  // namespace
 
@@ -46,7 +60,8 @@ StripPlan strip_plan(int fmt, int bits, int gs, int64_t rows, int64_t N, int64_t
   float best = 0.f;
   for (int ln = 0; ln < 3; ln++) {
     const int nwn = 1 << ln;
-    if (kWindow[lm][ln] == 0.f || (nwn_req > 0 && nwn != nwn_req)) continue;
+    const StripCost& c = kCost[lm][ln];
+    if (c.window == 0.f || (nwn_req > 0 && nwn != nwn_req)) continue;
     const int wps = strip_wps(mt, nwn), sr = (8 / nwn) * 128 * wps;
     if (sr < 2 * gs || strip_lds(mt, nwn, gs, experts) > kQmvLdsMax) continue;
     const int64_t blocks = (N + 16 * nwn - 1) / (16 * nwn);
@@ -55,15 +70,12 @@ StripPlan strip_plan(int fmt, int bits, int gs, int64_t rows, int64_t N, int64_t
     for (int64_t ks = ks_req > 0 && experts <= 0 ? ks_req : 1; ks <= ks_max; ks++) {
       const int64_t per_split = (steps + ks - 1) / ks;
       const int64_t ksr = (steps + per_split - 1) / per_split;
-      const float windows = (float)((per_split + 1) / 2 * 2 * wps) * passes;  // steps run in pairs
-      const float rounds = (float)(blocks * ksr * std::max<int64_t>(experts, 1)) / cus;
-      // a second launch adds the K ranges' partials
-      const float reduce = ksr > 1 ? 2.5f + (float)(ksr * rows * N) * 8.f / 4e6f : 0.f;
-      // a part-full last round costs most of a full one (12288 and 14336 x
-      // 4096 in 384 and 448 workgroups of 32 rows 19.5-19.8 us, 8192 x 4096 in
-      // 256 of them 10.6)
-      const float waves = rounds <= 1.f ? 1.f : 0.15f * rounds + 0.85f * std::ceil(rounds);
-      const float us = (kStart[lm][ln] + kWindow[lm][ln] * windows) * waves + reduce;
+      const int64_t windows = (per_split + 1) / 2 * 2 * wps;  // steps run in pairs
+      const float x = (float)(blocks * ksr * std::max<int64_t>(experts, 1)) / cus;
+      const float rounds = std::max(1.f, c.whole * std::ceil(x) + (1.f - c.whole) * x);
+      const bool narrow = N % (ksr > 1 ? 4 : 8) != 0;
+      const float us = kBitsCost[bits] * (c.start + rounds * passes * (c.pass + c.pass_fill * std::min(x, 1.f) + (narrow ? c.narrow : 0.f) + c.window * windows) +
+                                          (ksr > 1 ? c.sum + c.sum_each * (float)ksr * rows * N * 1e-6f : 0.f));
       if (p.ok && us >= best) continue;
       best = us;
       p.ok = true;
@@ -72,7 +84,8 @@ StripPlan strip_plan(int fmt, int bits, int gs, int64_t rows, int64_t N, int64_t
       p.row_blocks = (int)blocks;
       p.ks = (int)ksr;
       p.k_per_split = (int)std::min<int64_t>(per_split * sr, (int64_t)1 << 30);
-      p.windows = (int)windows;
+      p.windows = (int)(windows * passes);
+      p.us = us;
       p.lds = strip_lds(mt, nwn, gs, experts);
     }
   }

@@ -30,6 +30,29 @@ def _timed(monkeypatch, call, other):
     return graph_us([call, switched])
 
 
+def _dense(M, N, K, bits, gs, dt):
+    w, s, b = _matrix((N,), K, bits, gs)
+    x, s, b = (t.to(dt) for t in (torch.randn(M, K, device="cuda"), s, b))
+    return lambda: mq.quantized_matmul(x, w, s, b, True, gs, bits)
+
+
+@pytest.mark.parametrize("bits,M,N,K,gs", [(4, 78, 151936, 256, 32), (4, 97, 151936, 576, 64), (4, 52, 151936, 256, 128),
+                                           (8, 49, 151936, 1152, 128), (2, 831, 17072, 288, 32), (5, 739, 5645, 544, 32)])
+def test_strip_kernel_and_the_ones_it_replaces(monkeypatch, bits, M, N, K, gs):
+    # many rounds of strips with a short K, several passes over an odd width
+    announce("route time, strip", bits, M, N, K)
+    now, other = _timed(monkeypatch, _dense(M, N, K, bits, gs, torch.bfloat16), {"MLXQ_STRIP": "0"})
+    assert now <= 1.25 * other, (now, other)
+
+
+@pytest.mark.parametrize("bits,M,N,K,gs", [(3, 257, 155, 1024, 128), (6, 223, 142, 1152, 128), (3, 323, 146, 512, 64), (2, 488, 282, 512, 32)])
+def test_odd_widths_of_small_matrices(monkeypatch, bits, M, N, K, gs):
+    # the prefill tiles against the general kernel, which these switches leave the call to
+    announce("route time, odd widths", bits, M, N, K)
+    now, other = _timed(monkeypatch, _dense(M, N, K, bits, gs, torch.float16), {"MLXQ_QMM_MIN_ROWS": "100000", "MLXQ_STRIP": "0"})
+    assert now <= 1.25 * other, (now, other)
+
+
 @pytest.mark.parametrize("E,N,K,B,hot", [(128, 768, 2048, 8192, 8), (128, 768, 2048, 1024, 8), (32, 2048, 1024, 2048, 2)])
 def test_skewed_sorted_gather(monkeypatch, E, N, K, B, hot):
     # all entries on a few experts, against the grouped tiles
