@@ -277,44 +277,31 @@ float tile_us(int tile, bool odd, int64_t M, int64_t N, int nks, int ks, int num
          (ksr > 1 ? c.sum + c.sum_each * (float)ksr * M * N * 1e-6f : 0.f);
 }
 
-// Tile and K split of a grid that fits about one round of the CUs (129-1024
-// rows; the 2-, 3-, 5- and 6-bit codes, which have no 256 x 128 tile on 8
-// waves, at any row count).  One round of 256 x 128 tiles (3/4 to all of the
-// CUs) runs unsplit, else 0.58 to one round of 256 x 256 tiles does (14336 x
-// 4096: 512 rows 76 us, 768 rows 107).  Otherwise each tile with no split,
-// the split that fills the round and one less is priced as
-//   start + K-steps per workgroup * (c1 + c2 * fill) + partial sums
-// fitted to 300 graph-timed calls on MI355X (4- and 8-bit codes, seven
-// shapes, 129-1024 rows, 9% rms); over those the choice is within 1.3% of
-// the fastest (tile, split) on average, where splits by powers of two alone
-// were 10% off: 1900 x 1152 256 rows 16.2 us vs 20.5, 6144 x 4096 333 rows
-// 41.5 vs 47, 768 rows 62 vs 73, 4096 x 14336 768 rows 111 vs 134.
-int plan_mid(bool odd, int64_t M, int64_t N, int nks, int num_cus, int& ks_out) {
-  struct Cost {
-    int tile, slots, min_steps;  // workgroups per CU, K-steps a split keeps
-    float start, c1, c2;
-  };
-  constexpr Cost costs[3] = {{4, 1, 8, 14.7f, 1.474f, 0.10f}, {6, 2, 4, 9.6f, 0.583f, 0.677f}, {8, 1, 8, 10.4f, 0.831f, 0.286f}};
-  auto tiles_of = [&](int t) { return ((M + kBM[t] - 1) / kBM[t]) * ((N + kBN[t] - 1) / kBN[t]); };
-  ks_out = 1;
-  if (!odd && tiles_of(8) * 4 >= (int64_t)num_cus * 3 && tiles_of(8) <= num_cus) return 8;
-  if (tiles_of(4) * 100 >= (int64_t)num_cus * 58 && tiles_of(4) <= num_cus) return 4;
-  int best_tile = 6;
-  float best = 0.f;
-  for (const Cost& c : costs) {
-    if (odd && c.tile == 8) continue;
-    const int64_t tiles = tiles_of(c.tile), slots = (int64_t)c.slots * num_cus;
-    const int mx = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(slots / tiles, nks / c.min_steps), 16));
+// The cheapest tile and K split by that price, among each tile with no split,
+// the split that fills a round and one less, for a grid of up to about one
+// round (129-1024 rows; the 2-, 3-, 5- and 6-bit codes, which have tiles 4 and
+// 6 only, at any row count).  The plan whose splits are powers of two
+// (tile_in, ks_in; 0: none) is kept unless another is 3% cheaper.  Over 10900
+// timed calls at 129-1024 rows the choice is 2.5% off the fastest (tile, split)
+// measured, that plan 18%; 1% of them are more than 5% slower than on that
+// plan (4% with prices without the round's own time and the narrow rows: 4-bit
+// 469 rows over 17388 x 1152 64 us vs 50).
+int plan_mid(bool odd, int64_t M, int64_t N, int nks, int num_cus, int tile_in, int ks_in, int& ks_out) {
+  int best_tile = tile_in;
+  float best = ks_in > 0 ? 0.97f * tile_us(tile_in, odd, M, N, nks, ks_in, num_cus) : 0.f;
+  ks_out = ks_in;
+  for (int tile : {4, 6, 8}) {
+    if (odd && tile == 8) continue;
+    const int64_t tiles = ((M + kBM[tile] - 1) / kBM[tile]) * ((N + kBN[tile] - 1) / kBN[tile]);
+    const int64_t slots = (int64_t)(tile == 6 ? 2 : 1) * num_cus;
+    const int mx = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(slots / tiles, nks / 4), 16));
     for (int ks : {1, mx - 1, mx}) {
       if (ks < 1) continue;
-      const int steps = (nks + ks - 1) / ks, ksr = (nks + steps - 1) / steps;
-      const float x = (float)(tiles * ksr) / slots;
-      const float per = x <= 1.f ? c.c1 + c.c2 * x : (c.c1 + c.c2) * 0.5f * (std::ceil(x) + x);
-      const float us = c.start + per * steps + (ksr > 1 ? 2.5f + (float)ksr * M * N * 1e-6f : 0.f);
+      const float us = tile_us(tile, odd, M, N, nks, ks, num_cus);
       if (best > 0.f && us >= best) continue;
       best = us;
-      best_tile = c.tile;
-      ks_out = ksr;
+      best_tile = tile;
+      ks_out = ks;
     }
   }
   return best_tile;
@@ -346,7 +333,7 @@ QmmPlan qmm_plan(int fmt, int gs, int64_t M, int64_t N, int64_t K, int num_cus, 
   if (tile_req >= 0 && tile_req < kTiles) {
     tile = tile_req;
   } else if (odd) {
-    tile = plan_mid(true, M, N, nks, num_cus, ks_planned);
+    tile = plan_mid(true, M, N, nks, num_cus, 0, 0, ks_planned);
   } else {
     // 256 x 256 (8 waves) when there are enough tiles or K is long enough
     // for a K split to fill the CUs; else 128 x 128, two workgroups per CU.
@@ -365,7 +352,7 @@ QmmPlan qmm_plan(int fmt, int gs, int64_t M, int64_t N, int64_t K, int num_cus, 
     if (mid_rows && (K >= 8192 || one_round8)) tile = 8;
     else tile = (M > 128 && (tiles_of(4) >= num_cus / 2 || K >= 8192)) ? 4 : 6;
     if (fit_round && ksplit_req <= 0 && M > 128 && M <= 1024 && tiles_of(4) <= num_cus)
-      tile = plan_mid(false, M, N, nks, num_cus, ks_planned);
+      tile = plan_mid(false, M, N, nks, num_cus, tile, pow2_split(tile), ks_planned);
   }
   p.tile = tile;
   p.rows_per_tile = kBM[tile];

@@ -53,6 +53,16 @@ def test_odd_widths_of_small_matrices(monkeypatch, bits, M, N, K, gs):
     assert now <= 1.25 * other, (now, other)
 
 
+@pytest.mark.parametrize("bits,M,N,K,gs", [(4, 469, 17388, 1152, 128), (4, 462, 18864, 1024, 128), (4, 442, 17336, 448, 64)])
+def test_prefill_tiles_of_short_k(monkeypatch, bits, M, N, K, gs):
+    # the planned tile and K split against each tile unsplit
+    announce("route time, prefill tiles", bits, M, N, K)
+    call = _dense(M, N, K, bits, gs, torch.bfloat16)
+    for tile in ("4", "6", "8"):
+        now, other = _timed(monkeypatch, call, {"MLXQ_QMM_TILE": tile, "MLXQ_QMM_KSPLIT": "1"})
+        assert now <= 1.2 * other, (tile, now, other)
+
+
 @pytest.mark.parametrize("E,N,K,B,hot", [(128, 768, 2048, 8192, 8), (128, 768, 2048, 1024, 8), (32, 2048, 1024, 2048, 2)])
 def test_skewed_sorted_gather(monkeypatch, E, N, K, B, hot):
     # all entries on a few experts, against the grouped tiles
