@@ -370,9 +370,12 @@ struct StripPlan {
   int nwn = 4;             // waves along the weight rows (16 rows each)
   int row_blocks = 0, ks = 1, k_per_split = 0;
   int windows = 0;         // 128-position windows each wave multiplies
-  float us = 0.f;          // price of a dense launch
+  float us = 0.f;          // price of the launch (0: none known)
   size_t lds = 0;
 };
+// Mean number of passes of `rows` entries that an expert of `avg` entries on
+// average takes (at least 1; entries spread evenly, about normal)
+float mean_passes(double avg, int rows);
 StripPlan strip_plan(int fmt, int bits, int gs, int64_t rows, int64_t N, int64_t K, int64_t experts, int cus,
                      int nwn_req, int mt_req, int ks_req);
 hipError_t strip_launch(int fmt, int bits, const StripArgs& a, const StripPlan& p, hipStream_t stream);
@@ -458,6 +461,10 @@ inline int64_t qmm_sk_bytes(const QmmPlan& p) { return p.sk_len > 0 ? (int64_t)2
 int qmm_tile_rows(int tile);
 // Grouped gather: tiles along N for `tile`; tiles_m = segments is set by the caller.
 QmmPlan qmm_plan_grouped(int fmt, int gs, int64_t N, int64_t K, int tile);
+// its tile for `per` entries an expert on average, and the microseconds of a
+// gather of B entries of one row (index lists, grouping and tiles)
+constexpr int grouped_tile(int64_t per) { return per <= 64 ? 3 : per <= 128 ? 2 : 0; }
+float grouped_us(int bits, int64_t N, int64_t K, int64_t E, int64_t B, int cus);
 // tile_req / ksplit_req < 0 (or 0 for ksplit) choose by shape.
 // mix: allow the two-launch plan (tile2) when neither tile nor split is requested;
 // streamk: allow the stream-K plan there (it takes precedence).

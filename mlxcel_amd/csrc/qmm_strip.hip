@@ -36,7 +36,42 @@ constexpr StripCost kCost[5][3] = {
 // the same by width of the codes
 constexpr float kBitsCost[9] = {1.f, 1.f, 0.97f, 0.99f, 0.97f, 1.04f, 1.03f, 1.f, 1.f};
 
+
+// Microseconds of a sorted gather spread evenly over its experts:
+//   start + rounds * (round + passes * (pass + window * windows of a wave))
+// window for 4-bit codes, `bits8` more of it for 8-bit ones and `fill` more in
+// a full round.  Fitted to 5900 graph-timed calls on MI355X (8-256 experts of
+// N 64-5760, K 512-4096; 8-200 entries each), 8-18% rms.
+struct GatherCost {
+  int mt, nwn, slots;  // slots: workgroups per CU
+  float start, round, pass, narrow, window, bits8, fill, whole;
+};
+constexpr GatherCost kGather[] = {
+    {1, 4, 1, 5.3f, 0.0f, 1.4f, 0.2f, 0.24f, 0.85f, 1.28f, 0.68f}, {2, 2, 1, 3.1f, 0.1f, 2.3f, 0.4f, 0.76f, 0.12f, 0.48f, 0.50f},
+    {2, 4, 1, 4.4f, 0.0f, 1.3f, 0.3f, 0.72f, 0.25f, 0.03f, 0.59f}, {3, 2, 2, 2.2f, 0.6f, 2.9f, 0.5f, 1.23f, 0.15f, 0.62f, 0.50f},
+    {3, 4, 1, 5.4f, 0.5f, 1.2f, 0.6f, 0.88f, 0.52f, 0.00f, 0.65f}, {8, 4, 1, 3.1f, 2.1f, 1.2f, 0.4f, 1.71f, 0.00f, 0.70f, 0.63f}};
+
+float gather_us(int bits, int64_t N, int64_t B, int64_t E, const StripPlan& p, int cus) {
+  for (const GatherCost& c : kGather) {
+    if (c.mt != p.mt || c.nwn != p.nwn) continue;
+    const float x = (float)(E * p.row_blocks) / (float)(c.slots * cus);
+    const float rounds = std::max(1.f, c.whole * std::ceil(x) + (1.f - c.whole) * x);
+    const float window = c.window * (bits == 8 ? 1.f + c.bits8 : 1.f) * (1.f + c.fill * std::min(x, 1.f));
+    return c.start + rounds * (c.round + mean_passes((double)B / E, 16 * p.mt) * (c.pass + (N % 8 != 0 ? c.narrow : 0.f) + window * p.windows));
+  }
+  return 0.f;
+}
+
 }  // namespace
+
+float mean_passes(double avg, int rows) {
+  double sum = 1.0;  // P(more than j passes' entries) over j
+  for (int j = 1;; j++) {
+    const double more = 0.5 * (1.0 - std::erf((j * (double)rows + 0.5 - avg) / std::sqrt(2.0 * avg)));
+    sum += more;
+    if (more < 1e-3) return (float)sum;
+  }
+}
 
 StripPlan strip_plan(int fmt, int bits, int gs, int64_t rows, int64_t N, int64_t K, int64_t experts, int cus,
                      int nwn_req, int mt_req, int ks_req) {
@@ -56,7 +91,7 @@ StripPlan strip_plan(int fmt, int bits, int gs, int64_t rows, int64_t N, int64_t
   for (int i = 0; i < 5; i++)
     if (mt_req == kTilesM[i]) lm = i;
   const int mt = kTilesM[lm];
-  const int64_t passes = experts > 0 ? 1 : (rows + 16 * mt - 1) / (16 * mt);
+  const float passes = experts > 0 ? mean_passes((double)rows / experts, 16 * mt) : (float)((rows + 16 * mt - 1) / (16 * mt));
   float best = 0.f;
   for (int ln = 0; ln < 3; ln++) {
     const int nwn = 1 << ln;
@@ -84,11 +119,12 @@ StripPlan strip_plan(int fmt, int bits, int gs, int64_t rows, int64_t N, int64_t
       p.row_blocks = (int)blocks;
       p.ks = (int)ksr;
       p.k_per_split = (int)std::min<int64_t>(per_split * sr, (int64_t)1 << 30);
-      p.windows = (int)(windows * passes);
+      p.windows = (int)(experts > 0 ? windows : windows * (int64_t)passes);
       p.us = us;
       p.lds = strip_lds(mt, nwn, gs, experts);
     }
   }
+  if (p.ok && experts > 0) p.us = gather_us(bits, N, rows, experts, p, cus);
   if (p.ok && (p.row_blocks * (int64_t)16 * p.nwn >= ((int64_t)1 << 31) || p.ks > 65535 || experts > 65535)) p.ok = false;
   return p;
 }

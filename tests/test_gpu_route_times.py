@@ -63,6 +63,17 @@ def test_prefill_tiles_of_short_k(monkeypatch, bits, M, N, K, gs):
         assert now <= 1.2 * other, (tile, now, other)
 
 
+@pytest.mark.parametrize("E,N,K,B,bits", [(128, 2026, 640, 16328, 4), (60, 5641, 896, 3300, 8), (8, 5186, 1664, 928, 4), (64, 3282, 640, 3234, 8)])
+def test_evenly_routed_sorted_gather(monkeypatch, E, N, K, B, bits):
+    # many rounds of strips with a short K, against the grouped tiles
+    announce("route time, even gather", E, N, K, B, bits)
+    w, s, b = _matrix((E, N), K, bits, 128)
+    x = torch.randn(B, 1, K, device="cuda").to(torch.bfloat16)
+    ids = torch.randint(0, E, (B,), generator=torch.Generator().manual_seed(B)).sort().values.to(torch.int32).cuda()
+    now, tiles = _timed(monkeypatch, lambda: mq.gather_qmm(x, w, s, b, None, ids, True, 128, bits, "affine", True), {"MLXQ_STRIP": "0"})
+    assert now <= 1.2 * tiles, (now, tiles)
+
+
 @pytest.mark.parametrize("E,N,K,B,hot", [(128, 768, 2048, 8192, 8), (128, 768, 2048, 1024, 8), (32, 2048, 1024, 2048, 2)])
 def test_skewed_sorted_gather(monkeypatch, E, N, K, B, hot):
     # all entries on a few experts, against the grouped tiles
