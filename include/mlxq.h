@@ -107,8 +107,10 @@ typedef struct mlxq_array {
  * (2 x CUs x 256 KiB, 128 MiB on MI355X) takes the plan without stream-K
  * instead of allocating; its result then equals the eager call's within
  * rounding, not bit for bit (stream-K adds a cut tile's two K pieces in
- * fp32).  No counterpart in the reference (MLX allocates inside each
- * eval). */
+ * fp32).  So does a captured call of 5-128 rows, or of 129-1024 rows, whose K
+ * split needs more scratch than the stream holds where a plan of the same
+ * kernel needs none.  No counterpart in the reference (MLX allocates inside
+ * each eval). */
 mlxq_status mlxq_workspace_reserve(size_t bytes, void* stream);
 
 /* Bytes of device memory held by the workspaces (current and replaced

@@ -1382,6 +1382,14 @@ bool try_strip(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, cons
   const int fmt = sp.mode == MXFP4_M ? mlxq::MXFP4 : mlxq::AFF4;
   mlxq::StripPlan p = mlxq::strip_plan(fmt, sp.bits, sp.gs, rows, sp.N, sp.K, 0, cus, kn.strip_nwn, kn.strip_mt, kn.strip_ks);
   if (!p.ok || (!forced && !odd && rows > 64 && p.windows > 4)) return false;
+  auto part = [&](int ks) { return (size_t)ks * rows * sp.N * sizeof(float); };
+  // partials that cannot be had here (under capture, past the fixed scratch):
+  // one K range, which needs none.  Of 11600 timed calls of odd widths it is
+  // at 0.31-0.95 of the general kernel with its K split (5-16 rows over 8192
+  // weight rows and more 0.31, 65-128 over less than 2048 0.94), of 11700 calls
+  // of the others at 0.58-0.95 of the tiles with theirs
+  if (p.ks > 1 && !scratch_fits(dev, stream, part(p.ks), ss))
+    p = mlxq::strip_plan(fmt, sp.bits, sp.gs, rows, sp.N, sp.K, 0, cus, kn.strip_nwn, kn.strip_mt, 1);
   if (!forced) {
     // where the kernels below are priced lower they keep the call: the general
     // kernel many rows and small matrices (6-bit 1000 rows over 1100 x 544 28 us
@@ -1390,17 +1398,25 @@ bool try_strip(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, cons
     // over 151936 x 256 27 vs 80, 52 rows 26 vs 49; 8-bit 49 rows over 151936 x
     // 1152 72 vs 114).  Of 3100 timed calls at 5-128 rows 9 are more than 5%
     // slower than on the other kernel.
-    const float other = odd ? mlxq::gen_us(mlxq::gen_plan(rows, sp.N, sp.K, 1, cus, 0), rows, sp.N, cus)
-                            : mlxq::qmm_plan(fmt_of(sp.mode, sp.bits), sp.gs, rows, sp.N, sp.K, cus, -1, 0).us;
+    // (0: none, or its own partials cannot be had)
+    float other;
+    int other_ks;
+    if (odd) {
+      const mlxq::GenPlan gp = mlxq::gen_plan(rows, sp.N, sp.K, 1, cus, 0);
+      other = mlxq::gen_us(gp, rows, sp.N, cus);
+      other_ks = gp.ks;
+    } else {
+      const mlxq::QmmPlan qp = mlxq::qmm_plan(fmt_of(sp.mode, sp.bits), sp.gs, rows, sp.N, sp.K, cus, -1, 0);
+      other = qp.us;
+      other_ks = qp.ksplit;
+    }
+    if (other_ks > 1 && !scratch_fits(dev, stream, part(other_ks), ss)) other = 0.f;
     if (other > 0.f && p.us > other) return false;
     // mxfp4 rows that the tiles do not take (K not a multiple of 64) have the
     // skinny kernel, 9.6-11 us for up to 128 rows of small matrices where one
     // pass of strips takes 12
     if (sp.mode == MXFP4_M && sp.K % 64 != 0 && rows > 72 && sp.K < 1664 && sp.N <= 640) return false;
   }
-  auto part = [&] { return (size_t)p.ks * rows * sp.N * sizeof(float); };
-  // partials that cannot be had here: the kernels below
-  if (p.ks > 1 && !scratch_fits(dev, stream, part(), ss)) return false;
   mlxq::StripArgs a{};
   a.x = static_cast<const uint16_t*>(x->data);
   a.w = static_cast<const uint32_t*>(w->data);
@@ -1412,7 +1428,7 @@ bool try_strip(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, cons
   a.N = (int)sp.N;
   a.K = (int)sp.K;
   a.gs_shift = gs_shift_of(sp.gs);
-  if (p.ks > 1) a.ws = reinterpret_cast<float*>(workspace(dev, stream, part(), ss));
+  if (p.ks > 1) a.ws = reinterpret_cast<float*>(workspace(dev, stream, part(p.ks), ss));
   hip_check(mlxq::strip_launch(fmt, sp.bits, a, p, stream), "qmm_strip launch");
   if (p.ks > 1)
     hip_check(mlxq::launch_splitk_reduce(a.ws, a.out, rows * sp.N, p.ks, stream, a.xt), "reduce launch");

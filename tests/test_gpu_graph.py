@@ -11,7 +11,8 @@ import torch
 
 import mlxcel_amd as mq
 import oracle as orc
-from helpers import TOL, affine_case, announce, dev_bf16, dev_u32, dev_u8, host_u16, max_rel, mxfp4_case, setknob
+from helpers import (TOL, affine_case, announce, dev_bf16, dev_u32, dev_u8, host_u16, kernels_of, max_rel, mxfp4_case,
+                     setknob)
 
 pytestmark = pytest.mark.gpu
 
@@ -195,3 +196,65 @@ def test_capture_with_strided_x_after_a_reserve():
     assert mq.get_cache_memory() == held
     junk = torch.randn(1 << 20, device="cuda")
     replay_and_check(g, out, eager, lambda: junk.mul_(0.25))
+
+
+def _random(M, N, K, bits, gs, dt):
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    w = torch.randint(-2 ** 31, 2 ** 31, (N, K * bits // 32), generator=g, device="cuda").to(torch.int32).view(torch.uint32)
+    s = (torch.rand(N, K // gs, generator=g, device="cuda") * 0.01 + 0.002).to(dt)
+    return torch.randn(M, K, generator=g, device="cuda").to(dt), w, s, -8 * s
+
+
+@pytest.mark.parametrize("bits,M,N,K,dt,plan", [
+    (3, 8, 256, 14336, torch.bfloat16, {"MLXQ_STRIP": "2", "MLXQ_STRIP_KS": "1"}),
+    (6, 100, 1024, 14336, torch.float16, {"MLXQ_STRIP": "2", "MLXQ_STRIP_KS": "1"}),
+    (4, 32, 512, 14336, torch.bfloat16, {"MLXQ_STRIP": "2", "MLXQ_STRIP_KS": "1"}),
+    (4, 768, 6144, 4096, torch.float16, {"MLXQ_QMM_TILE": "8", "MLXQ_QMM_KSPLIT": "1"})])
+def test_captured_k_splits_without_scratch(monkeypatch, bits, M, N, K, dt, plan):
+    # the K split of the eager call has no scratch here: the captured call takes
+    # the plan of the same kernel that needs none, bit for bit
+    announce("graph_no_scratch", bits, M, N, K)
+    X, W, S, B = _random(M, N, K, bits, 64, dt)
+    names = kernels_of(lambda: mq.quantized_matmul(X, W, S, B, True, 64, bits))
+    assert len(names) == 2, names  # the eager call is split: a kernel and the sum of its partials
+    with monkeypatch.context() as m:
+        for k, v in plan.items():
+            setknob(m, k, v)
+        want = mq.quantized_matmul(X, W, S, B, True, 64, bits)
+    setknob(monkeypatch, "MLXQ_NONE", "")
+    out = torch.empty(M, N, dtype=dt, device="cuda")
+    st = torch.cuda.Stream()  # never used: its workspace is empty
+    torch.cuda.synchronize()
+    held = mq.get_cache_memory()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        mq.quantized_matmul(X, W, S, B, True, 64, bits, out=out)
+    assert mq.get_cache_memory() == held
+    junk = torch.randn(1 << 20, device="cuda")
+    for rep in range(3):
+        out.zero_()
+        junk.mul_(0.5)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), rep
+
+
+def test_captured_odd_width_prefill_without_scratch_gets_a_status():
+    # tiles and general kernel both split K here
+    announce("graph_no_scratch odd prefill")
+    M, N, K = 256, 256, 8192
+    X, W, S, B = _random(M, N, K, 6, 64, torch.bfloat16)
+    out = torch.zeros(M, N, dtype=torch.bfloat16, device="cuda")
+    g = torch.cuda.CUDAGraph()
+    err = None
+    with torch.cuda.graph(g, stream=torch.cuda.Stream()):
+        try:
+            mq.quantized_matmul(X, W, S, B, True, 64, 6, out=out)
+        except mq.ops.QuantizedOpError as e:
+            err = str(e)
+        out.add_(1.0)
+    assert err is not None and "captured" in err, err
+    g.replay()
+    torch.cuda.synchronize()
+    assert float(out.float().min()) == 1.0 == float(out.float().max())

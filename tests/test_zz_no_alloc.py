@@ -81,6 +81,23 @@ def test_noalloc_rejects_calls_beyond_its_scratch(monkeypatch):
     assert float(out.float().abs().max()) == 0.0  # nothing ran
 
 
+def test_noalloc_strips_beyond_its_scratch(monkeypatch):
+    # 16 forced K ranges of 128 rows need 128 MiB of partials: one range instead
+    setknob(monkeypatch, "MLXQ_STRIP", "2")
+    setknob(monkeypatch, "MLXQ_STRIP_KS", "1")
+    announce("noalloc_strip")
+    M, N, K = 128, 16384, 4096
+    X, W, S, B = case(M, N, K, 3150)
+    want = host_u16(mq.quantized_matmul(X, W, S, B, True, 64, 4))
+    setknob(monkeypatch, "MLXQ_STRIP_KS", "16")
+    out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    st = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    assert noalloc(X, W, S, B, out, st) == _lib.OK, _lib.last_error()
+    st.synchronize()
+    np.testing.assert_array_equal(host_u16(out), want)
+
+
 # Run in a fresh process, so the captured call is the first call into the
 # library there: the device address of the fixed scratch is resolved while
 # the stream is being captured.
