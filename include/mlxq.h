@@ -150,8 +150,10 @@ const char* mlxq_version(void);
  * (x, scales, biases and result) 4/8-bit affine with transpose=true (decode
  * and prefill; its prefill dequantizes the weights to float16, as the
  * reference's dequantize + GEMM route does).  Affine codes of 2, 3, 5 and 6
- * bits with bfloat16 or float16 x, scales and biases of one type and
- * transpose=true run the specialised kernels from 5 rows on.  Every other
+ * bits with bfloat16 or float16 x, scales and biases of one type, 2-D weights
+ * and transpose=true run the specialised kernels from 5 rows on (up to 1024
+ * rows where K is not a multiple of 64), except small matrices that the
+ * general path runs faster.  Every other
  * combination runs the general path: affine calls of 1-4 rows per matrix with transpose=true
  * (1-2 with transpose=false) on its row-streaming decode kernels (fp32
  * products, no weight rounding), the rest on its tile kernel (float16

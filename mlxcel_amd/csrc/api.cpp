@@ -1295,9 +1295,11 @@ bool strip_types(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* scale
   return sp.mode == MXFP4_M && sp.gs == 32 && sp.bits == 4 && dt == MLXQ_BFLOAT16;
 }
 
-// float16 prefill (rows >= MLXQ_QMM_MIN_ROWS once the mid-size kernels have
-// declined): the 32x32-MFMA tile kernel's float16 instantiation; a requested
-// tile of the 16x16-MFMA kernel (bfloat16 only) falls back to the planner's.
+// Prefill on the 32x32-MFMA tile kernel of calls that are not the specialised
+// bfloat16 ones: float16 4- and 8-bit codes (rows >= MLXQ_QMM_MIN_ROWS once the
+// mid-size kernels have declined), and codes of 2, 3, 5 and 6 bits of either
+// 16-bit type past 128 rows.  K a multiple of 64.  A requested tile of the
+// 16x16-MFMA kernel (bfloat16 only) falls back to the planner's.
 bool try_qmm_tile(const QmmSpec& sp, const mlxq_array* x, const mlxq_array* w, const mlxq_array* scales,
                   const mlxq_array* biases, mlxq_array* out, int64_t rows, hipStream_t stream, const ScratchSrc& ss) {
   const bool odd = sp.mode == AFFINE && sp.bits != 4 && sp.bits != 8;
