@@ -22,13 +22,15 @@
 // distinct banks.  Weights never touch LDS: a ring of RD windows per wave is
 // in flight in registers.
 //
-// What bounds it (MI355X, 14336 x 4096, 3-bit g64, 8 rows, 14.6 us, 62.6 on
-// the general tile kernel; timing-only copies): 7.4 us are left with the
-// dequantization, the staging and the weight stream all taken out (launch,
-// first loads, sum over the K waves), the dequantization (2.6 VALU per code)
-// adds 2.5, staging and barriers 2; the 25.7 MB of weights (3.2 us at 8 TB/s)
-// hide under these.  Per 128-position window a wave spends 0.70 us at 16
-// activation rows, 0.98 at 32, 1.10 at 48, 1.21 at 64 and 2.4 at 128.  Two windows per
+// What bounds it (MI355X, 14336 x 4096, 3-bit g64, 8 rows, 13.8 us, 62.6 on
+// the general tile kernel; timing-only copies with 32 weight rows per workgroup,
+// 14.6 us, where 64 are taken now): 7.4 us are left with the dequantization, the
+// staging and the weight stream all taken out (launch, first loads, sum over the
+// K waves), the dequantization (2.6 VALU per code) adds 2.5, staging and barriers
+// 2; the 25.7 MB of weights (3.2 us at 8 TB/s) hide under these.  Per
+// 128-position window a wave spends 0.64 us at 16 activation rows, 0.82 at 32,
+// 1.05 at 48, 1.12 at 64 and 1.84 at 128 (64 weight rows per workgroup; the
+// planner's table in qmm_strip.hip has the others).  Two windows per
 // step (one past 16 rows) and a ring of two steps measured best of 1, 2 and
 // 4 windows and rings of 2 to 8; two workgroups per CU instead of one
 // changed nothing.
@@ -201,9 +203,11 @@ __global__ __launch_bounds__(512, 2) void qmm_strip_kernel(const StripArgs a) {
     }
   }
   // A dense call's expert and first row stay values in registers: with them
-  // folded away the compiler schedules some of the kernels worse (float16 2-bit,
-  // 64 rows of 14336 x 4096 at 64 weight rows a workgroup 13-17% slower, bfloat16
-  // 3-bit at 8 rows 5%, others up to 8% faster).
+  // folded away the compiler schedules the kernels differently, some worse
+  // (float16 2-bit 64 rows 13-17% slower at 64 weight rows a workgroup, bfloat16
+  // 3-bit 8-16 rows 4-7%) and some better (bfloat16 2-6-bit 128 rows 18-26%
+  // faster, float16 3-5-bit 48 rows 7-10%, float16 6-bit 8-16 rows 24% over
+  // 14336 x 4096 and equal over 4096 x 4096 and 4096 x 14336).
   if constexpr (!GATHER) {
     asm volatile("" : "+s"(e));
     asm volatile("" : "+s"(first));
